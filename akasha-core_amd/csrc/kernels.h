@@ -110,6 +110,10 @@ struct GemmParams {
   // and a flag set to 1 when a result is not finite.
   const uint16_t* bp16;
   int* range_flag;
+  // launch_gemm_h3: A's fp16 planes (split_rows_f16_bytes), and for GEMM_SILU
+  // the planes its output goes to (the next GEMM's A) instead of c.
+  const uint16_t* ap16;
+  uint16_t* cp16;
   // GEMM_QKV on ragged prompts packed back to back: row m is position
   // rowmap[m].y of sequence rowmap[m].x (instead of m / S, m % S).
   const int2* rowmap;
@@ -124,7 +128,12 @@ struct GemmParams {
   // tile.  Null: no split.
   float* split_ws;
   int* split_cnt;
-  int split_kc;  // set by launch_gemm: rows of K per split
+  int split_kc;  // set by the launchers: rows of K per split
+  // launch_gemm_h3 with GEMM_ADD: a buffer of kGemmPartsFloats.  Where
+  // gemm_h3_splits(M, N, K) > 1 the partial sums of that many K ranges are
+  // stored to parts[z][M][N] instead of being added to c, for the next
+  // launch_rows_rmsnorm to add.  Null: c is always complete.
+  float* parts;
 };
 
 enum { FLASH_X6 = 1, FLASH_H3 = 2, FLASH_FP32 = 3 };  // FlashParams::x6
@@ -142,6 +151,7 @@ struct FlashParams {
   const akh_flash_attn_meta* meta;  // per-shader path: S, dim, scale and
                                     // row_offset come from it (1 sequence)
   uint16_t* o16;  // launch_flash_bf16: bfloat16 output (o unused)
+  uint16_t* op16;  // flash_writes_planes: fp16 planes of the output (o unused)
   int x6;         // launch_flash, head_dim 64 / 128: split-bfloat16 MFMAs
                   // (fp32 accuracy) instead of fp32 MFMAs; FLASH_H3: split
                   // fp16 MFMAs (fp32 accuracy), setting *range_flag when an
@@ -162,8 +172,12 @@ struct FlashParams {
 hipError_t launch_gemm(const GemmParams& p, int epi, hipStream_t s);
 hipError_t launch_flash(const FlashParams& p, int batch, int max_rows,
                         hipStream_t s);
-hipError_t launch_rows_rmsnorm(const float* x, const float* w, float* out,
-                               int rows, int size, float eps, hipStream_t s);
+// With nparts > 0 (size % 4 == 0, size <= kNormPartsMax) x first takes the
+// sum of the partial sums parts[z][rows][size]; out may then be null.
+constexpr int kNormPartsMax = 4096;
+hipError_t launch_rows_rmsnorm(float* x, const float* w, float* out, int rows, int size,
+                               float eps, hipStream_t s, const float* parts = nullptr,
+                               int nparts = 0);
 
 // The optional bfloat16-MFMA prefill: bfloat16 MFMA operands (round to
 // nearest even), fp32 accumulation, fp32 residual stream and KV cache.
@@ -181,7 +195,25 @@ hipError_t launch_gemm_x6(const GemmParams& p, int epi, hipStream_t s);
 // per multiply-add.  Sets *p.range_flag when a result is not finite (an
 // operand beyond fp16's range); the caller then recomputes in fp32.  K % 8 == 0.
 hipError_t launch_gemm_h3(const GemmParams& p, int epi, hipStream_t s);
-// The fp16 planes of a [K, N] row-major matrix for launch_gemm_h3 (K * N * 4 bytes).
+// K ranges whose partial sums launch_gemm_h3 stores to p.parts (1: none).
+// They take at most one 64 x 64 tile per CU and split.
+constexpr int kGemmPartsMax = 8;
+constexpr size_t kGemmPartsFloats = 256 * 64 * 64;
+int gemm_h3_splits(int M, int N, int K);
+// The fp16 planes of a [K, N] row-major matrix for launch_gemm_h3.
+size_t split_weights_f16_bytes(int K, int N);
+// The fp16 planes of `rows` rows of K floats, launch_gemm_h3's A, and the
+// producers that write them: the row norm (size % 8 == 0, size <=
+// kNormPartsMax), flash attention of these shapes (FlashParams::op16), GEMM_SILU
+// and a conversion of fp32 rows.
+size_t split_rows_f16_bytes(size_t rows, int K);
+hipError_t launch_rows_rmsnorm_planes(float* x, const float* w, uint16_t* planes, int rows,
+                                      int size, float eps, hipStream_t s,
+                                      const float* parts = nullptr, int nparts = 0);
+hipError_t launch_rows_planes(const float* x, int rows, int K, uint16_t* planes, hipStream_t s);
+inline bool flash_writes_planes(const FlashParams& p) {
+  return p.x6 == FLASH_H3 && (p.hd == 64 || p.hd == 128);
+}
 hipError_t launch_split_weights_f16(const float* w, int K, int N, uint16_t* wp, hipStream_t s);
 // wt[n, k] = w[k, n] for a [K, N] row-major matrix.
 hipError_t launch_transpose_f32(const float* w, int K, int N, float* wt, hipStream_t s);

@@ -30,17 +30,22 @@ __global__ void k_embedding_rows(const uint32_t* tokens, const float* table,
 // Rows of up to 4096 floats (a multiple of 4): one wave per row, four rows
 // per block, the row held in registers between the sum of squares (a wave
 // butterfly, no LDS or barrier) and the scaling, read and written 16 bytes
-// at a time.  Other sizes: one block per row, element by element.
-template <int QL>  // float4 per lane: size <= 256 QL
-__global__ __launch_bounds__(256) void k_rows_rmsnorm(const float* __restrict__ x,
+// at a time.  PARTS (these sizes only): the row is first the sum of x and the
+// nparts partial sums of the GEMM before it (parts[z][row][:], added in order,
+// then to x), which is stored back to x; out may then be null for the sum
+// alone (an instantiation of its own: its registers would halve the waves of
+// the plain norm).  Other sizes: one block per row, element by element.
+template <int QL, bool PARTS = false>  // float4 per lane: size <= 256 QL
+__global__ __launch_bounds__(256) void k_rows_rmsnorm(float* __restrict__ x,
                                                       const float* __restrict__ w,
                                                       float* __restrict__ out, int rows,
-                                                      int size, float eps) {
+                                                      int size, float eps,
+                                                      const float* __restrict__ parts,
+                                                      int nparts) {
   if (QL > 0) {
     const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (row >= rows) return;
-    const float4* xr = reinterpret_cast<const float4*>(x + (size_t)row * size);
-    float4* o = reinterpret_cast<float4*>(out + (size_t)row * size);
+    float4* xr = reinterpret_cast<float4*>(x + (size_t)row * size);
     const float4* g4 = reinterpret_cast<const float4*>(w);
     const int nq = size >> 2;
     float4 v[QL > 0 ? QL : 1], g[QL > 0 ? QL : 1];
@@ -49,9 +54,42 @@ __global__ __launch_bounds__(256) void k_rows_rmsnorm(const float* __restrict__ 
     for (int i = 0; i < QL; ++i) {
       const int q = lane + 64 * i;
       v[i] = q < nq ? xr[q] : make_float4(0.f, 0.f, 0.f, 0.f);
-      g[i] = q < nq ? g4[q] : make_float4(0.f, 0.f, 0.f, 0.f);
-      ss += v[i].x * v[i].x + v[i].y * v[i].y + v[i].z * v[i].z + v[i].w * v[i].w;
+      g[i] = out && q < nq ? g4[q] : make_float4(0.f, 0.f, 0.f, 0.f);
     }
+    if (PARTS) {
+      constexpr int NB = QL <= 4 ? 4 : 2;  // partial sums per batch of loads
+      float4 sum[QL > 0 ? QL : 1];
+#pragma unroll
+      for (int i = 0; i < QL; ++i) sum[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+      for (int z = 0; z < nparts; z += NB) {
+        float4 t[NB][QL > 0 ? QL : 1];
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+          const float4* pr =
+              reinterpret_cast<const float4*>(parts + ((size_t)(z + b) * rows + row) * size);
+#pragma unroll
+          for (int i = 0; i < QL; ++i) {
+            const int q = lane + 64 * i;
+            t[b][i] = z + b < nparts && q < nq ? pr[q] : make_float4(0.f, 0.f, 0.f, 0.f);
+          }
+        }
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+          for (int i = 0; i < QL; ++i) add4(sum[i], t[b][i]);
+      }
+#pragma unroll
+      for (int i = 0; i < QL; ++i) {
+        const int q = lane + 64 * i;
+        add4(v[i], sum[i]);
+        if (q < nq) xr[q] = v[i];
+      }
+      if (!out) return;
+    }
+    float4* o = reinterpret_cast<float4*>(out + (size_t)row * size);
+#pragma unroll
+    for (int i = 0; i < QL; ++i)
+      ss += v[i].x * v[i].x + v[i].y * v[i].y + v[i].z * v[i].z + v[i].w * v[i].w;
     ss = wave_sum(ss);
     const float rs = 1.0f / sqrtf(ss / (float)size + eps);
 #pragma unroll
@@ -157,26 +195,27 @@ __device__ __forceinline__ void epi_pair_gemm(const GemmParams& p, int M,
 }
 
 // The epilogue of one 32-row MFMA tile pair as a lane holds it: rows
-// mbase + acc_row(r, h), r = 0..15, columns n and n + 1 (n even).  Every load
+// mbase + acc_row(r, h), r = r0 .. r0 + NR - 1, columns n and n + 1 (n even).  Every load
 // the epilogue needs (the residual of GEMM_ADD, the RoPE table and row map of
-// GEMM_QKV) is issued for all 16 rows before the first store: stores may
+// GEMM_QKV) is issued for all rows before the first store: stores may
 // alias those loads as far as the compiler knows, so pair by pair each load
 // would wait out the previous store and its own latency in turn.
-template <int EPI>
+template <int EPI, int NR = 16>
 __device__ __forceinline__ void epi_tile(const GemmParams& p, int M, int N, int mbase, int n,
-                                         const float (&v0)[16], const float (&v1)[16]) {
+                                         const float (&v0)[NR], const float (&v1)[NR],
+                                         int r0 = 0) {
   const int h = (threadIdx.x & 63) >> 5;
   if (EPI == GEMM_ADD && (N & 1) == 0 && n < N) {
-    float2 old[16];
+    float2 old[NR];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int m = mbase + acc_row(r, h);
+    for (int r = 0; r < NR; ++r) {
+      const int m = mbase + acc_row(r0 + r, h);
       old[r] = m < M ? *reinterpret_cast<const float2*>(p.c + (size_t)m * N + n)
                      : make_float2(0.f, 0.f);
     }
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int m = mbase + acc_row(r, h);
+    for (int r = 0; r < NR; ++r) {
+      const int m = mbase + acc_row(r0 + r, h);
       if (m < M)
         *reinterpret_cast<float2*>(p.c + (size_t)m * N + n) =
             make_float2(old[r].x + v0[r], old[r].y + v1[r]);
@@ -186,10 +225,10 @@ __device__ __forceinline__ void epi_tile(const GemmParams& p, int M, int N, int 
   if (EPI == GEMM_QKV && n < N) {
     const int dim = p.dim, region = n / dim, c = n - region * dim;
     const int i = (c % p.head_dim) >> 1, half_hd = p.head_dim >> 1;
-    int seq[16], t[16];
+    int seq[NR], t[NR];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int m = min(mbase + acc_row(r, h), M - 1);
+    for (int r = 0; r < NR; ++r) {
+      const int m = min(mbase + acc_row(r0 + r, h), M - 1);
       if (p.rowmap) {
         const int2 st = p.rowmap[m];
         seq[r] = st.x;
@@ -198,14 +237,14 @@ __device__ __forceinline__ void epi_tile(const GemmParams& p, int M, int N, int 
         div_rows(m, p.S, seq[r], t[r]);
       }
     }
-    float2 cs[16];
+    float2 cs[NR];
     if (region < 2) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) cs[r] = p.rope[(size_t)t[r] * half_hd + i];
+      for (int r = 0; r < NR; ++r) cs[r] = p.rope[(size_t)t[r] * half_hd + i];
     }
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int m = mbase + acc_row(r, h);
+    for (int r = 0; r < NR; ++r) {
+      const int m = mbase + acc_row(r0 + r, h);
       if (m >= M) continue;
       float a = v0[r], b = v1[r];
       if (region < 2) rope_pair(a, b, cs[r].x, cs[r].y);
@@ -222,7 +261,7 @@ __device__ __forceinline__ void epi_tile(const GemmParams& p, int M, int N, int 
     return;
   }
 #pragma unroll
-  for (int r = 0; r < 16; ++r) epi_pair_gemm<EPI>(p, M, N, mbase + acc_row(r, h), n, v0[r], v1[r]);
+  for (int r = 0; r < NR; ++r) epi_pair_gemm<EPI>(p, M, N, mbase + acc_row(r0 + r, h), n, v0[r], v1[r]);
 }
 
 // C[M,N] = A[M,K] B[K,N], 128x128 block tile, BK = 16, 4 waves in 2x2,
@@ -875,33 +914,33 @@ __global__ __launch_bounds__(256) void k_transpose_f32(const float* __restrict__
   }
 }
 
-// The fp16 planes of k_gemm_h3's weights: for a [K, N] row-major matrix,
-// wp[((n K/8 + k/8) 2 + p) 8 + k%8] = plane p (0: hi, 1: lo) of w[k, n] as
-// split by split2_f16, so one 32-byte run holds the hi and lo octets of
-// eight consecutive k of column n.  K % 8 == 0.  A 32 x 32 tile through LDS;
-// thread (n, octet) writes its 32 bytes.
+// The fp16 planes of a [K, N] row-major matrix for the split-fp16 GEMMs
+// (x = hi + 2^-11 lo, split2_f16) in MFMA fragment order: columns in groups of
+// 64, K in steps of 32 (both padded with zeros), each group's step 8 KB of
+// eight fragments [u][t][plane] of 1 KB, u the 16-k half, t the column parity,
+// plane hi then lo.  Lane (j, h) of a fragment owns the 16 bytes at 16 (32 h +
+// j): the eight k 16 u + 8 h .. + 7 of column 2 j + t (adjacent columns in the
+// two tiles of one lane, for the paired epilogues).  A wave's fragment is so
+// one contiguous kilobyte, in memory and in LDS.  One block per group and step.
 __global__ __launch_bounds__(256) void k_split_weights_f16(const float* __restrict__ w, int K,
                                                            int N, uint16_t* __restrict__ wp) {
-  __shared__ float t[32][33];
-  const int k0 = blockIdx.y * 32, n0 = blockIdx.x * 32;
-  const int c = threadIdx.x & 31, r = threadIdx.x >> 5;
-  for (int i = r; i < 32; i += 8) {
-    const int k = k0 + i, n = n0 + c;
-    t[i][c] = (k < K && n < N) ? w[(size_t)k * N + n] : 0.f;
+  __shared__ float t[32][65];
+  const int k0 = blockIdx.y * 32, n0 = blockIdx.x * 64;
+  for (int i = threadIdx.x; i < 32 * 64; i += 256) {
+    const int k = k0 + (i >> 6), n = n0 + (i & 63);
+    t[i >> 6][i & 63] = (k < K && n < N) ? w[(size_t)k * N + n] : 0.f;
   }
   __syncthreads();
-  if (threadIdx.x >= 128) return;
-  const int nl = threadIdx.x >> 2, q = threadIdx.x & 3;
-  const int n = n0 + nl, k = k0 + 8 * q;
-  if (n >= N || k >= K) return;
-  const float4 x0 = make_float4(t[8 * q][nl], t[8 * q + 1][nl], t[8 * q + 2][nl], t[8 * q + 3][nl]);
-  const float4 x1 =
-      make_float4(t[8 * q + 4][nl], t[8 * q + 5][nl], t[8 * q + 6][nl], t[8 * q + 7][nl]);
+  const int j = threadIdx.x & 31, h = (threadIdx.x >> 5) & 1, ut = threadIdx.x >> 6;
+  const int c = 2 * j + (ut & 1), kk = 16 * (ut >> 1) + 8 * h;
+  const float4 x0 = make_float4(t[kk][c], t[kk + 1][c], t[kk + 2][c], t[kk + 3][c]);
+  const float4 x1 = make_float4(t[kk + 4][c], t[kk + 5][c], t[kk + 6][c], t[kk + 7][c]);
   uint4 hi, lo;
   split2_f16(x0, x1, hi, lo);
-  uint4* dst = reinterpret_cast<uint4*>(wp + ((size_t)n * (K / 8) + k / 8) * 16);
+  uint4* dst = reinterpret_cast<uint4*>(wp) + ((size_t)blockIdx.x * gridDim.y + blockIdx.y) * 512 +
+               ut * 128 + 32 * h + j;
   dst[0] = hi;
-  dst[1] = lo;
+  dst[64] = lo;
 }
 
 // C[M,N] = A[M,K] B[K,N] in fp32 accuracy on v_mfma_f32_32x32x16_bf16.
@@ -1141,41 +1180,135 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_x6(GemmParams p) {
     }
 }
 
-// C[M,N] = A[M,K] B[K,N] in fp32 accuracy on v_mfma_f32_32x32x16_f16.  Each
-// fp32 element enters LDS as two fp16 terms (split2_f16: x = hi + 2^-11 lo,
-// to within 2^-22 |x|): A is split while it is staged, the weights once, into
-// fp16 planes (p.bp16, k_split_weights_f16), so their staging is a plain
-// copy.  A product takes three MFMAs: hi.hi into one accumulator, hi.lo +
-// lo.hi into a second, summed as acc + 2^-11 acc' at the end; the dropped
-// lo.lo term is below 2^-22 |a b|.  So a product costs 3 x 32 MFMA cycles per
-// 16 k (6 x 32 on k_gemm_x6) and four LDS fragments (six).  An operand beyond
-// fp16's range (|x| >= 65520) becomes an infinite hi, which makes every sum
-// it enters infinite or NaN: a block with a non-finite result sets
-// *p.range_flag, and the caller recomputes on the fp32 kernels (non-finite
-// inputs flag too, and come out the same there).
-//
-// Block tile BM x BN, BK = 32, waves WM (rows) x WN (columns), each owning
-// (BM / WM) x 64 as TA x 2 MFMA tiles.  Staging reads whole 128-byte lines:
-// piece f of a step is row f / 8, bytes 16 (f % 8) .. + 15 of that row's
-// step, so eight consecutive lanes read one row's line (loads that scatter
-// a wave over 32 rows, as in k_gemm_x6, ran at half the speed: the vector
-// cache serves a wave's lines one by one).  A B row's 128 bytes are the hi
-// and lo planes of its four k-octets, at the byte offset of the same k in
-// an fp32 [N, K] matrix.  LDS holds both planes of both operands k-contiguous
-// (rows of 32 k padded to 80 bytes: 16-byte fragment reads of 8 consecutive
-// rows hit distinct banks), double buffered; the global loads of step s + 2
-// are issued before step s + 1 is stored.  K % 8 == 0.
-template <int EPI, int BM, int BN, int WM, int WN>
-__global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_h3(GemmParams p) {
-  constexpr int BK = 32, LD = BK + 8, NT = 64 * WM * WN, NU = BK / 16;
-  constexpr int TA = BM / WM / 32;
-  static_assert(BN == 64 * WN && BM % (32 * WM) == 0, "wave tiles are (32 TA) x 64");
-  constexpr int PR = BK / 4;  // 16-byte pieces per row and step
-  constexpr int FA = PR * BM / NT, FB = PR * BN / NT;
-  static_assert(FA >= 1 && FB >= 1 && FA * NT == PR * BM && FB * NT == PR * BN,
-                "every thread stages whole pieces of both operands");
-  __shared__ __align__(16) uint16_t As[2][2][BM][LD];
-  __shared__ __align__(16) uint16_t Bs[2][2][BN][LD];
+// ---------------------------------------------------------------------------
+// The split-fp16 GEMMs: C[M,N] = A[M,K] B[K,N] in fp32 accuracy on
+// v_mfma_f32_32x32x16_f16.  Each fp32 element is two fp16 terms (split2_f16:
+// x = hi + 2^-11 lo, to within 2^-22 |x|), A's written by the kernel that
+// produces it, the weights' once at upload, both as planes in MFMA fragment
+// order: K in steps of 32 (zeros past K), each step of 32 rows of A 4 KB of
+// four fragments [u][plane], of 64 columns of B 8 KB of eight ([u][t][plane],
+// k_split_weights_f16).  A product takes three MFMAs: hi.hi into one
+// accumulator, hi.lo + lo.hi into a second, summed as acc + 2^-11 acc' at the
+// end; the dropped lo.lo term is below 2^-22 |a b|.  An operand beyond fp16's
+// range (|x| >= 65520) has an infinite hi, which makes every sum it enters
+// infinite or NaN: a block with a non-finite result sets *p.range_flag, and
+// the caller recomputes on the fp32 kernels (non-finite inputs flag too, and
+// come out the same there).  Rows of A's last 32-row tile past M are whatever
+// the buffer holds; they reach only rows of C past M.
+// ---------------------------------------------------------------------------
+
+// The 16-byte piece (hi plane; lo is 64 pieces on) of row m, k-octet o in the
+// planes of A with `steps` 32-k steps.
+__device__ __forceinline__ size_t plane_piece(int m, int o, int steps) {
+  return (((size_t)(m >> 5) * steps + (o >> 2)) * 4 + ((o >> 1) & 1) * 2) * 64 + (o & 1) * 32 +
+         (m & 31);
+}
+
+// Element (m, c) of A's planes (`steps` 32-k steps), for producers whose lanes
+// do not hold octets.
+__device__ __forceinline__ void put_plane(uint16_t* planes, int m, int c, int steps, float v) {
+  const uint32_t hi = cvt_pk_f16(v, 0.f);
+  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+  const float r = (v - (float)__builtin_bit_cast(h2, hi)[0]) * 2048.f;
+  uint16_t* dst = planes + plane_piece(m, c >> 3, steps) * 8 + (c & 7);
+  dst[0] = (uint16_t)hi;
+  dst[512] = (uint16_t)cvt_pk_f16(r, 0.f);
+}
+
+// SiLU of a lane's rows r0 .. r0 + NR - 1 of columns n, n + 1 (as epi_tile's)
+// into the planes of the next GEMM's A (p.cp16, N its K).  A quad of lanes
+// holds four rows of one column octet; after a 4 x 4 exchange each lane holds
+// one row's octet, and a wave's stores cover whole 128-byte lines.
+template <int NR>
+__device__ __forceinline__ void epi_silu_planes(const GemmParams& p, int M, int N, int mbase,
+                                                int n, const float (&v0)[NR],
+                                                const float (&v1)[NR], int r0 = 0) {
+  static_assert(NR % 4 == 0, "whole row quads");
+  const int lane = threadIdx.x & 63, h = lane >> 5, i = lane & 3;
+  const int steps = (N + 31) / 32, o = n >> 3;
+  auto silu = [](float v) {
+    return v * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(v * -1.44269504088896341f));
+  };
+  auto dpp1 = [](uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, true);
+  };
+  auto dpp2 = [](uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, true);
+  };
+  // Lane i of a quad gets row i's words of lanes 0..3.
+  auto exchange = [&](const uint32_t (&x)[4]) {
+    uint32_t a[2][2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const uint32_t got = dpp1(i & 1 ? x[2 * q] : x[2 * q + 1]);
+      a[q][0] = i & 1 ? got : x[2 * q];
+      a[q][1] = i & 1 ? x[2 * q + 1] : got;
+    }
+    const uint32_t g0 = dpp2(i & 2 ? a[0][0] : a[1][0]), g1 = dpp2(i & 2 ? a[0][1] : a[1][1]);
+    return i & 2 ? make_uint4(g0, g1, a[1][0], a[1][1]) : make_uint4(a[0][0], a[0][1], g0, g1);
+  };
+#pragma unroll
+  for (int q = 0; q < NR / 4; ++q) {
+    uint32_t hi[4], lo[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+      const float a = silu(v0[4 * q + r]), b = silu(v1[4 * q + r]);
+      hi[r] = cvt_pk_f16(a, b);
+      const h2 hv = __builtin_bit_cast(h2, hi[r]);
+      lo[r] = cvt_pk_f16((a - (float)hv[0]) * 2048.f, (b - (float)hv[1]) * 2048.f);
+    }
+    const uint4 hp = exchange(hi), lp = exchange(lo);
+    const int m = mbase + 2 * (r0 + 4 * q) + 4 * h + i;  // acc_row(r0 + 4 q + i, h)
+    if (m < M && (o >> 2) < steps) {
+      uint4* dst = reinterpret_cast<uint4*>(p.cp16) + plane_piece(m, o, steps);
+      dst[0] = hp;
+      dst[64] = lp;
+    }
+  }
+}
+
+// The epilogue of a lane's rows r0 .. r0 + NR - 1 of a tile pair.
+template <int EPI, int NR>
+__device__ __forceinline__ bool epi_h3(const GemmParams& p, int M, int N, int mbase, int n,
+                                       const float (&v0)[NR], const float (&v1)[NR],
+                                       int r0 = 0) {
+  bool finite = true;
+#pragma unroll
+  for (int r = 0; r < NR; ++r)
+    finite = finite && ((__builtin_isfinite(v0[r]) && __builtin_isfinite(v1[r])) ||
+                        mbase + acc_row(r0 + r, (threadIdx.x & 63) >> 5) >= M);
+  if constexpr (EPI == GEMM_SILU)
+    epi_silu_planes<NR>(p, M, N, mbase, n, v0, v1, r0);
+  else
+    epi_tile<EPI, NR>(p, M, N, mbase, n, v0, v1, r0);
+  return finite;
+}
+
+// Block tile BM x BN of 64 x 64 wave tiles (WM x WN waves), K dealt to KG wave
+// groups (step s to group s % KG) whose sums meet in LDS at the end.  Each
+// group's steps stream through ST LDS buffers by buffer_load .. lds: a
+// fragment is a contiguous kilobyte on both sides, so staging takes no
+// registers, no address arithmetic per lane and no LDS bank conflicts, and
+// ST - 1 steps are in flight.  One barrier per step: past it the step's
+// pieces have landed (every wave waited for its own) and the buffer of the
+// step before has no reader left, so the next loads may be issued into it.
+// grid.z as k_gemm_h3k's.  What bounds it is the matrix pipe at the clock this
+// work runs at and the LDS beside it (a 256 x 128 step reads 128 KB and writes
+// 48 KB of LDS per 1536 MFMA cycles).  Against staging through registers with
+// A split in every block, us on MI355X: 8192 x 768 x 3072 134 -> 113, 16384 x
+// 6144 x 2048 1343 -> 1079, 16384 x 2048 x 8192 1696 -> 1354 (1218 TFLOP/s of
+// fp16 products; a plain 8192^3 bf16 library product runs at 1194).
+template <int EPI, int BM, int BN, int WM, int WN, int KG, int ST>
+__global__ __launch_bounds__(64 * WM * WN * KG, 2) void k_gemm_h3(GemmParams p) {
+  constexpr int NW = WM * WN, CA = BM / 32 * 4, CB = BN / 64 * 8, CH = (CA + CB) / NW;
+  static_assert(BN == 64 * WN && BM == 64 * WM, "wave tiles are 64 x 64");
+  static_assert(CA % NW == 0 && CB % NW == 0, "every wave stages whole fragments");
+  static_assert(KG == 1 || KG == 2, "one or two wave groups");
+  constexpr int STAGE = (CA + CB) * 1024;
+  constexpr int RED = KG > 1 ? NW * KG * 8192 : 0;
+  constexpr int BYTES = KG * ST * STAGE > RED ? KG * ST * STAGE : RED;
+  __shared__ __align__(16) unsigned char lds[BYTES];
 
   const int M = p.M, N = p.N, K = p.K;
   // Each XCD takes a contiguous run of tiles (see k_gemm_bf16).
@@ -1183,139 +1316,399 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_h3(GemmParams p) {
   const int per_xcd = (int)(gridDim.x * gridDim.y) / 8;
   if (id < per_xcd * 8) id = (id % 8) * per_xcd + id / 8;
   const int m0 = (id / gridDim.x) * BM, n0 = (id % gridDim.x) * BN;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave / WN, wn = wave % WN;
-  const int j = lane & 31, h = lane >> 5;
+  const int z = blockIdx.z;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int kg = wave / NW, w = wave % NW, wm = w / WN, wn = w % WN;
+  const int j = lane & 31;
+  // Steps [s0, s1) of K: all of them, or z's range (whole steps).
+  const int steps = (K + 31) / 32, s0 = z * p.split_kc / 32;
+  const int s1 = min(steps, s0 + (p.split_kc + 31) / 32), iters = (s1 - s0 + KG - 1) / KG;
 
-  // Loads go through buffer resources bounded to the block's rows of A and
-  // of the planes: pieces past M or N fall outside them, pieces past K get
-  // an offset outside them, and the hardware returns zeros for both.  B's
-  // LDS row L = 64 g + 32 t + jj holds column 64 g + 2 jj + t of the block
-  // (lane j of column tile t then reads column 2j + t: adjacent column pairs
-  // for the paired epilogues).
-  float4 ra[2][FA], rb[2][FB];
-  const __amdgpu_buffer_rsrc_t rsa = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<float*>(p.a + (size_t)m0 * K), (short)0, min(M - m0, BM) * K * 4, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rsb = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint16_t*>(p.bp16 + (size_t)n0 * K * 2), (short)0, min(N - n0, BN) * K * 4,
-      0x00020000);
-  auto ld4 = [](__amdgpu_buffer_rsrc_t rs, uint32_t vo) {
-    typedef float f4 __attribute__((ext_vector_type(4)));
-    const f4 v = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)vo, 0, 0));
-    return make_float4(v.x, v.y, v.z, v.w);
+  // Row tiles and column groups past the end are clamped to the last.
+  const int rt_last = min((M + 31) / 32 - m0 / 32, BM / 32) - 1;
+  const int cg_last = min((N + 63) / 64 - n0 / 64, BN / 64) - 1;
+  typedef int i4 __attribute__((ext_vector_type(4)));
+  auto rsrc = [](const void* base) {
+    const uint64_t v = (uint64_t)base;
+    return i4{(int)(uint32_t)v, (int)(uint32_t)(v >> 32), (int)0xFFFFFFFFu, 0x00020000};
   };
-  auto bcol = [](int L) { return (L & ~63) | ((L & 31) << 1) | ((L >> 5) & 1); };
-  auto gload = [&](int k0, int set) {
+  const i4 rsa = rsrc(p.ap16 + (size_t)(m0 / 32) * steps * 2048);
+  const i4 rsb = rsrc(p.bp16 + (size_t)(n0 / 64) * steps * 4096);
+  const uint32_t base =
+      (uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char*)lds + kg * ST * STAGE;
+  const uint32_t vo = lane * 16;
+  auto issue = [&](int step, int buf) {
 #pragma unroll
-    for (int i = 0; i < FA; ++i) {
-      const int f = tid + NT * i, r = f / PR, q = f % PR;
-      const uint32_t vo = k0 + 4 * q < K ? (uint32_t)(r * K + k0 + 4 * q) * 4u : 0x80000000u;
-      ra[set][i] = ld4(rsa, vo);
-    }
-#pragma unroll
-    for (int i = 0; i < FB; ++i) {
-      // Piece q of a B row: plane q % 2 of k-octet q / 2.
-      const int f = tid + NT * i, L = f / PR, q = f % PR;
-      const uint32_t vo =
-          k0 + 8 * (q >> 1) < K ? (uint32_t)(bcol(L) * K + k0) * 4u + 16u * q : 0x80000000u;
-      rb[set][i] = ld4(rsb, vo);
-    }
-  };
-  auto lstore = [&](int buf, int set) {
-    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-#pragma unroll
-    for (int i = 0; i < FA; ++i) {
-      const int f = tid + NT * i, r = f / PR, q = f % PR;
-      const float4 x = ra[set][i];
-      const uint32_t h0 = cvt_pk_f16(x.x, x.y), h1 = cvt_pk_f16(x.z, x.w);
-      const h2 a0 = __builtin_bit_cast(h2, h0), a1 = __builtin_bit_cast(h2, h1);
-      const uint32_t l0 = cvt_pk_f16((x.x - (float)a0[0]) * 2048.f, (x.y - (float)a0[1]) * 2048.f);
-      const uint32_t l1 = cvt_pk_f16((x.z - (float)a1[0]) * 2048.f, (x.w - (float)a1[1]) * 2048.f);
-      *reinterpret_cast<uint2*>(&As[buf][0][r][4 * q]) = make_uint2(h0, h1);
-      *reinterpret_cast<uint2*>(&As[buf][1][r][4 * q]) = make_uint2(l0, l1);
-    }
-#pragma unroll
-    for (int i = 0; i < FB; ++i) {
-      const int f = tid + NT * i, L = f / PR, q = f % PR;
-      *reinterpret_cast<float4*>(&Bs[buf][q & 1][L][8 * (q >> 1)]) = rb[set][i];
+    for (int i = 0; i < CH; ++i) {
+      const int c = i * NW + w;
+      const bool is_a = i * NW < CA;
+      const int f = is_a ? c : c - CA;
+      const uint32_t so =
+          is_a ? ((uint32_t)min(f >> 2, rt_last) * steps + step) * 4096u + (f & 3) * 1024u
+               : ((uint32_t)min(f >> 3, cg_last) * steps + step) * 8192u + (f & 7) * 1024u;
+      const uint32_t dst = base + buf * STAGE + c * 1024;
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                   :
+                   : "s"(dst), "v"(vo), "s"(is_a ? rsa : rsb), "s"(so)
+                   : "memory");
     }
   };
 
-  f32x16 acc[TA][2], cor[TA][2];
+  f32x16 acc[2][2], cor[2][2];
 #pragma unroll
-  for (int a = 0; a < TA; ++a)
+  for (int a = 0; a < 2; ++a)
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       acc[a][t] = zero16();
       cor[a][t] = zero16();
     }
-  // One step: fragments of both 16-k halves of buffer `buf`, then the MFMAs.
-  auto step = [&](int buf) {
-    f16x8 f[NU][2 + TA][2];  // [0..1]: B column tiles, [2 + a]: A row tiles
+  auto compute = [&](int buf) {
+    const unsigned char* st = lds + (kg * ST + buf) * STAGE + lane * 16;
+    f16x8 fa[2][2][2], fb[2][2][2];  // [u][row tile or column tile][plane]
 #pragma unroll
-    for (int u = 0; u < NU; ++u) {
+    for (int u = 0; u < 2; ++u) {
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int pl = 0; pl < 2; ++pl)
+          fa[u][a][pl] = f16x8_of(*reinterpret_cast<const uint4*>(
+              st + ((2 * wm + a) * 4 + u * 2 + pl) * 1024));
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int pl = 0; pl < 2; ++pl)
-          f[u][t][pl] = f16x8_of(*reinterpret_cast<const uint4*>(
-              &Bs[buf][pl][wn * 64 + t * 32 + j][16 * u + 8 * h]));
-#pragma unroll
-      for (int a = 0; a < TA; ++a)
-#pragma unroll
-        for (int pl = 0; pl < 2; ++pl)
-          f[u][2 + a][pl] = f16x8_of(*reinterpret_cast<const uint4*>(
-              &As[buf][pl][wm * (32 * TA) + a * 32 + j][16 * u + 8 * h]));
+          fb[u][t][pl] = f16x8_of(*reinterpret_cast<const uint4*>(
+              st + (CA + wn * 8 + (u * 2 + t) * 2 + pl) * 1024));
     }
+    // Every read of the step is issued before its first MFMA (left alone, the
+    // compiler reads four registers, waits for them, and reads the next).
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int u = 0; u < NU; ++u)
+    for (int u = 0; u < 2; ++u)
 #pragma unroll
-      for (int a = 0; a < TA; ++a) {
+      for (int a = 0; a < 2; ++a) {
 #pragma unroll
-        for (int t = 0; t < 2; ++t) cor[a][t] = mfma_f16(f[u][2 + a][1], f[u][t][0], cor[a][t]);
+        for (int t = 0; t < 2; ++t) cor[a][t] = mfma_f16(fa[u][a][1], fb[u][t][0], cor[a][t]);
 #pragma unroll
-        for (int t = 0; t < 2; ++t) cor[a][t] = mfma_f16(f[u][2 + a][0], f[u][t][1], cor[a][t]);
+        for (int t = 0; t < 2; ++t) cor[a][t] = mfma_f16(fa[u][a][0], fb[u][t][1], cor[a][t]);
 #pragma unroll
-        for (int t = 0; t < 2; ++t) acc[a][t] = mfma_f16(f[u][2 + a][0], f[u][t][0], acc[a][t]);
+        for (int t = 0; t < 2; ++t) acc[a][t] = mfma_f16(fa[u][a][0], fb[u][t][0], acc[a][t]);
       }
   };
 
-  // Step s computes on LDS buffer s % 2 after storing step s + 1 (register
-  // set (s + 1) % 2, loaded a step earlier) into the other buffer and issuing
-  // the loads of step s + 2 into set s % 2.  Steps past the end load zeros.
-  const int nk = (K + BK - 1) / BK;
-  gload(0, 0);
-  gload(BK, 1);
-  lstore(0, 0);
-  __syncthreads();
-  auto stepk = [&](int s, int buf) {
-    __builtin_amdgcn_sched_barrier(0);
-    gload((s + 2) * BK, buf);
-    __builtin_amdgcn_sched_barrier(0);
-    lstore(1 - buf, 1 - buf);
-    step(buf);
-    __syncthreads();
-  };
-  int s = 0;
-  for (; s + 2 <= nk; s += 2) {
-    stepk(s, 0);
-    stepk(s + 1, 1);
-  }
-  if (s < nk) stepk(s, 0);
-
-  bool finite = true;
+  auto step_of = [&](int it) { return s0 + it * KG + kg; };
 #pragma unroll
-  for (int a = 0; a < TA; ++a) {
+  for (int i = 0; i < ST - 1; ++i)
+    if (step_of(i) < s1) issue(step_of(i), i);
+  int buf = 0;
+  for (int it = 0; it < iters; ++it) {
+    // This step's pieces have landed; with three buffers the next step's may
+    // still be in flight.
+    if (ST > 2 && step_of(it + 1) < s1)
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(CH) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" : : : "memory");
+    __builtin_amdgcn_s_barrier();
+    const int nbuf = buf == 0 ? ST - 1 : buf - 1;  // the buffer of step it - 1
+    if (step_of(it + ST - 1) < s1) issue(step_of(it + ST - 1), nbuf);
+    if (KG == 1 || step_of(it) < s1) compute(buf);
+    buf = buf == ST - 1 ? 0 : buf + 1;
+  }
+
+  p.c += (size_t)z * M * N;
+  const int mw = m0 + wm * 64, n = n0 + wn * 64 + 2 * j;
+  bool finite = true;
+  auto value = [&](int a, int t, int r) { return acc[a][t][r] + cor[a][t][r] * 0x1p-11f; };
+  if constexpr (KG == 1) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      float v0[16], v1[16];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        v0[r] = value(a, 0, r);
+        v1[r] = value(a, 1, r);
+      }
+      finite = epi_h3<EPI, 16>(p, M, N, mw + 32 * a, n, v0, v1) && finite;
+    }
+  } else {
+    // Group kg finishes row tile kg: it takes the other group's sums of it.
+    float* red = reinterpret_cast<float*>(lds) + lane * 4;
+    __syncthreads();
     float v0[16], v1[16];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      v0[r] = acc[a][0][r] + cor[a][0][r] * 0x1p-11f;
-      v1[r] = acc[a][1][r] + cor[a][1][r] * 0x1p-11f;
-      finite = finite && __builtin_isfinite(v0[r]) && __builtin_isfinite(v1[r]);
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const float4 v = make_float4(value(a, t, 4 * q), value(a, t, 4 * q + 1),
+                                       value(a, t, 4 * q + 2), value(a, t, 4 * q + 3));
+          if (a != kg)
+            *reinterpret_cast<float4*>(red + ((a * NW + w) * 8 + t * 4 + q) * 256) = v;
+          else if (t == 0) {
+            v0[4 * q] = v.x, v0[4 * q + 1] = v.y, v0[4 * q + 2] = v.z, v0[4 * q + 3] = v.w;
+          } else {
+            v1[4 * q] = v.x, v1[4 * q + 1] = v.y, v1[4 * q + 2] = v.z, v1[4 * q + 3] = v.w;
+          }
+        }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float4 x = *reinterpret_cast<const float4*>(red + ((kg * NW + w) * 8 + q) * 256);
+      const float4 y = *reinterpret_cast<const float4*>(red + ((kg * NW + w) * 8 + 4 + q) * 256);
+      v0[4 * q] += x.x, v0[4 * q + 1] += x.y, v0[4 * q + 2] += x.z, v0[4 * q + 3] += x.w;
+      v1[4 * q] += y.x, v1[4 * q + 1] += y.y, v1[4 * q + 2] += y.z, v1[4 * q + 3] += y.w;
     }
-    epi_tile<EPI>(p, M, N, m0 + wm * (32 * TA) + a * 32, n0 + wn * 64 + 2 * j, v0, v1);
-    }
+    finite = epi_h3<EPI, 16>(p, M, N, mw + 32 * kg, n, v0, v1);
+  }
   if (!finite) *p.range_flag = 1;
+}
+
+// The same for grids of few rows, where k_gemm_h3's block tiles leave most
+// CUs idle and each block walks all of K on its own: a block owns 32 TR rows x
+// 64 columns and its W waves deal the 16-k units of K among themselves, so the
+// chain of dependent loads is W times shorter and one barrier per block
+// remains (the waves' sums meet in LDS).  A wave reads its fragments straight
+// from memory; D units are in flight per wave.  Wave w takes units 2 w, 2 w +
+// 1, then those 2 W further.  With grid.z > 1 each z takes p.split_kc k and
+// stores its partial sums to p.c + z M N (GEMM_STORE; the caller's next norm
+// adds them).  Waves add in order, so results are reproducible.  At 64 rows it
+// is bound by a few memory round trips in a row: 64 x 2304 x 768 26 us on 128
+// x 128 tiles, 7.9 here; 64 x 768 x 3072 88 and 6.5 (8 ranges).
+template <int EPI, int TR, int W, int D>
+__global__ __launch_bounds__(64 * W, 2) void k_gemm_h3k(GemmParams p) {
+  static_assert(D % 2 == 0 && W >= 4 * TR, "whole pairs of units in flight; four rows per wave");
+  __shared__ __align__(16) float red[W][TR * 2][4][64][4];
+
+  const int M = p.M, N = p.N, K = p.K;
+  // Each XCD takes a contiguous run of (split, column group, row tile), row
+  // tiles fastest: one XCD reads a column group's weights once.
+  const int gm = gridDim.x, gn = gridDim.y;
+  int id = blockIdx.x + gm * (blockIdx.y + gn * blockIdx.z);
+  const int total = gm * gn * gridDim.z, per_xcd = total / 8;
+  if (id < per_xcd * 8) id = (id % 8) * per_xcd + id / 8;
+  const int z = id / (gm * gn), rem = id - z * (gm * gn);
+  const int g = rem / gm, m0 = (rem - g * gm) * (32 * TR);
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int j = lane & 31;
+  const int k0 = z * p.split_kc, k1 = min(K, k0 + p.split_kc);  // k0 % 32 == 0
+
+  // Units past the range and row tiles past M are read from the last one (a
+  // unit's products are skipped then, a row tile's rows never stored).
+  const int steps = (K + 31) / 32, u0 = k0 / 16, u1 = (k1 + 15) / 16;
+  const int rt_last = (M + 31) / 32 - 1;
+  const uint4* ag[TR];
+#pragma unroll
+  for (int a = 0; a < TR; ++a)
+    ag[a] = reinterpret_cast<const uint4*>(p.ap16) +
+            (size_t)min(m0 / 32 + a, rt_last) * steps * 256 + lane;
+  const uint4* bg = reinterpret_cast<const uint4*>(p.bp16) + (size_t)g * steps * 512 + lane;
+  uint4 ra[D][TR][2], rb[D][4];
+  auto load = [&](int u, int set) {
+    const size_t c = min(u, u1 - 1);
+#pragma unroll
+    for (int a = 0; a < TR; ++a)
+#pragma unroll
+      for (int pl = 0; pl < 2; ++pl) ra[set][a][pl] = ag[a][c * 128 + 64 * pl];
+#pragma unroll
+    for (int f = 0; f < 4; ++f) rb[set][f] = bg[c * 256 + 64 * f];
+  };
+  f32x16 acc[TR][2], cor[TR][2];
+#pragma unroll
+  for (int a = 0; a < TR; ++a)
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      acc[a][t] = zero16();
+      cor[a][t] = zero16();
+    }
+  auto mul = [&](int set) {
+#pragma unroll
+    for (int a = 0; a < TR; ++a) {
+      const f16x8 ah = f16x8_of(ra[set][a][0]), al = f16x8_of(ra[set][a][1]);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) cor[a][t] = mfma_f16(al, f16x8_of(rb[set][2 * t]), cor[a][t]);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) cor[a][t] = mfma_f16(ah, f16x8_of(rb[set][2 * t + 1]), cor[a][t]);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) acc[a][t] = mfma_f16(ah, f16x8_of(rb[set][2 * t]), acc[a][t]);
+    }
+  };
+  auto unit = [&](int i) { return u0 + 2 * ((i >> 1) * W + w) + (i & 1); };
+#pragma unroll
+  for (int i = 0; i < D; ++i) load(unit(i), i);
+  for (int i = 0; unit(i) < u1; i += D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      if (unit(i + d) < u1) mul(d);
+      load(unit(i + D + d), d);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+
+  // Every wave's sums to LDS, then wave w adds four rows of tile pair w / 4
+  // over the waves and runs their epilogue.
+#pragma unroll
+  for (int a = 0; a < TR; ++a)
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<float4*>(red[w][2 * a + t][q][lane]) =
+            make_float4(acc[a][t][4 * q] + cor[a][t][4 * q] * 0x1p-11f,
+                        acc[a][t][4 * q + 1] + cor[a][t][4 * q + 1] * 0x1p-11f,
+                        acc[a][t][4 * q + 2] + cor[a][t][4 * q + 2] * 0x1p-11f,
+                        acc[a][t][4 * q + 3] + cor[a][t][4 * q + 3] * 0x1p-11f);
+  __syncthreads();
+  if (w >= 4 * TR) return;
+  const int a = w >> 2, q = w & 3;
+  float v0[4] = {0.f, 0.f, 0.f, 0.f}, v1[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < W; ++i) {
+    const float4 x = *reinterpret_cast<const float4*>(red[i][2 * a][q][lane]);
+    const float4 y = *reinterpret_cast<const float4*>(red[i][2 * a + 1][q][lane]);
+    v0[0] += x.x, v0[1] += x.y, v0[2] += x.z, v0[3] += x.w;
+    v1[0] += y.x, v1[1] += y.y, v1[2] += y.z, v1[3] += y.w;
+  }
+  p.c += (size_t)z * M * N;
+  if (!epi_h3<EPI, 4>(p, M, N, m0 + 32 * a, g * 64 + 2 * j, v0, v1, 4 * q)) *p.range_flag = 1;
+}
+
+// k_rows_rmsnorm with its rows into A's planes: a wave per row, eight rows per
+// block, lane l the octets l, l + 64, ..  The eight rows' pieces of an octet
+// and plane are one 128-byte line: they meet in LDS and leave as whole lines
+// (stored by each wave for itself, 16 bytes per line, 8192 x 768 took 31 us).
+// size % 8 == 0, size <= 512 QO.
+template <int QO, bool PARTS>
+__global__ __launch_bounds__(512) void k_rows_rmsnorm_planes(float* __restrict__ x,
+                                                             const float* __restrict__ w,
+                                                             uint16_t* __restrict__ planes,
+                                                             int rows, int size, float eps,
+                                                             const float* __restrict__ parts,
+                                                             int nparts) {
+  // Piece (octet o, plane, row r) at 16 (9 (2 o + plane) + r): the odd stride
+  // spreads a wave's octets over the banks.
+  __shared__ __align__(16) uint4 pieces[QO * 64 * 2 * 9];
+  const int row0 = blockIdx.x * 8, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int row = min(row0 + wave, rows - 1);  // past the end: the last row again, not stored
+  const bool live = row0 + wave < rows;
+  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+  float* xr0 = x + (size_t)row * size;
+  float4* xr = reinterpret_cast<float4*>(xr0);
+  // A row's loads go through a buffer resource of its own size, so lanes past
+  // it read zeros without a branch (written as conditionals, each float of
+  // these loads became a load and a branch: 8192 x 768 took 27 us).
+  auto rsrc = [&](const float* p) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p), (short)0, size * 4,
+                                             0x00020000);
+  };
+  auto ld4 = [](__amdgpu_buffer_rsrc_t rs, int q) {
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    const f4 v = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(rs, q * 16, 0, 0));
+    return make_float4(v.x, v.y, v.z, v.w);
+  };
+  const __amdgpu_buffer_rsrc_t rx = rsrc(xr0), rg = rsrc(w);
+  const int no = size >> 3, steps = (size + 31) / 32;
+  float4 v[QO][2], g[QO][2];
+#pragma unroll
+  for (int i = 0; i < QO; ++i)
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int o = lane + 64 * i;
+      v[i][e] = ld4(rx, 2 * o + e);
+      g[i][e] = ld4(rg, 2 * o + e);
+    }
+  if (PARTS) {
+    constexpr int NB = QO <= 2 ? 4 : 2;  // partial sums per batch of loads
+    float4 sum[QO][2];
+#pragma unroll
+    for (int i = 0; i < QO; ++i) sum[i][0] = sum[i][1] = zero;
+    for (int z = 0; z < nparts; z += NB) {
+      float4 t[NB][QO][2];
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        // Past nparts: the last one again, not added.
+        const __amdgpu_buffer_rsrc_t rp =
+            rsrc(parts + ((size_t)min(z + b, nparts - 1) * rows + row) * size);
+#pragma unroll
+        for (int i = 0; i < QO; ++i)
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            const int o = lane + 64 * i;
+            t[b][i][e] = ld4(rp, 2 * o + e);
+          }
+      }
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        if (z + b >= nparts) break;
+#pragma unroll
+        for (int i = 0; i < QO; ++i) {
+          add4(sum[i][0], t[b][i][0]);
+          add4(sum[i][1], t[b][i][1]);
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < QO; ++i) {
+      const int o = lane + 64 * i;
+      add4(v[i][0], sum[i][0]);
+      add4(v[i][1], sum[i][1]);
+      if (live && o < no) {
+        xr[2 * o] = v[i][0];
+        xr[2 * o + 1] = v[i][1];
+      }
+    }
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < QO; ++i)
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+      ss += v[i][e].x * v[i][e].x + v[i][e].y * v[i][e].y + v[i][e].z * v[i][e].z +
+            v[i][e].w * v[i][e].w;
+  ss = wave_sum(ss);
+  const float rs = 1.0f / sqrtf(ss / (float)size + eps);
+#pragma unroll
+  for (int i = 0; i < QO; ++i) {
+    const int o = lane + 64 * i;
+    if (o >= 4 * steps) continue;  // octets past the row are zeros
+    float4 y[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+      y[e] = make_float4(__fmul_rn(__fmul_rn(v[i][e].x, rs), g[i][e].x),
+                         __fmul_rn(__fmul_rn(v[i][e].y, rs), g[i][e].y),
+                         __fmul_rn(__fmul_rn(v[i][e].z, rs), g[i][e].z),
+                         __fmul_rn(__fmul_rn(v[i][e].w, rs), g[i][e].w));
+    uint4 hi, lo;
+    split2_f16(y[0], y[1], hi, lo);
+    pieces[(2 * o) * 9 + wave] = hi;
+    pieces[(2 * o + 1) * 9 + wave] = lo;
+  }
+  __syncthreads();
+  const int r = threadIdx.x & 7, m = row0 + r;
+  if (m >= rows) return;
+  for (int q = threadIdx.x >> 3; q < 8 * steps; q += 64)  // q = 2 octet + plane
+    reinterpret_cast<uint4*>(planes)[plane_piece(m, q >> 1, steps) + 64 * (q & 1)] =
+        pieces[q * 9 + r];
+}
+
+// fp32 rows into A's planes, one 16-byte piece of each plane per thread (for
+// producers that write fp32 rows only).  K % 8 == 0.
+__global__ __launch_bounds__(256) void k_rows_planes(const float* __restrict__ x, int rows, int K,
+                                                     uint16_t* __restrict__ planes) {
+  const int steps = (K + 31) / 32;
+  const long e = (long)blockIdx.x * 256 + threadIdx.x;
+  const int m = (int)(e / (steps * 4)), o = (int)(e % (steps * 4));
+  if (m >= rows) return;
+  uint4 hi = make_uint4(0, 0, 0, 0), lo = hi;
+  if (8 * o < K) {
+    const float4* src = reinterpret_cast<const float4*>(x + (size_t)m * K + 8 * o);
+    split2_f16(src[0], src[1], hi, lo);
+  }
+  uint4* dst = reinterpret_cast<uint4*>(planes) + plane_piece(m, o, steps);
+  dst[0] = hi;
+  dst[64] = lo;
 }
 
 // Causal flash attention with bfloat16 MFMAs (head_dim 64 or 128), the
@@ -1965,12 +2358,32 @@ __device__ __forceinline__ bool flash_h3_tile(const FlashParams& p, unsigned cha
   }
   float (*Os)[33] = reinterpret_cast<float (*)[33]>(lds + wave * 32 * 33 * 4);
   float* op = p.o + fs.o + hh * hd;
+  const int row0 = p.op16 ? (int)(fs.o / d) : 0;
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < 16; ++r) Os[j][acc_row(r, h)] = o[t][r] * inv;
     __syncthreads();
+    if (p.op16) {
+      // A's planes of out_proj (hd == HD): lane j a row, four octets a tile.
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const int oc = 2 * e + h, qrow = q0 + wave * 32 + j;
+        if (qrow >= S) continue;
+        uint4 hi, lo;
+        split2_f16(make_float4(Os[j][8 * oc], Os[j][8 * oc + 1], Os[j][8 * oc + 2],
+                               Os[j][8 * oc + 3]),
+                   make_float4(Os[j][8 * oc + 4], Os[j][8 * oc + 5], Os[j][8 * oc + 6],
+                               Os[j][8 * oc + 7]),
+                   hi, lo);
+        uint4* dst = reinterpret_cast<uint4*>(p.op16) +
+                     plane_piece(row0 + qrow, (hh * HD + 32 * t) / 8 + oc, d / 32);
+        dst[0] = hi;
+        dst[64] = lo;
+      }
+      continue;
+    }
     for (int e = lane; e < 32 * 32; e += 64) {
       const int r = e >> 5, c = e & 31;
       const int qrow = q0 + wave * 32 + r;
@@ -2237,6 +2650,7 @@ __device__ __forceinline__ void flash_x6w_tile(const FlashParams& p, unsigned ch
   if (h == 0) ML[wave * 32 + j] = make_float2(mrow, lrow);
   __syncthreads();
   float* op = p.o + fs.o + hh * HD;
+  const int row0 = p.op16 ? (int)(fs.o / d) : 0;
   for (int e = tid; e < 32 * HD; e += 64 * NW) {
     const int qr = e / HD, dim = e % HD, qrow = q0 + qr;
     if (qrow >= S) continue;
@@ -2254,7 +2668,10 @@ __device__ __forceinline__ void flash_x6w_tile(const FlashParams& p, unsigned ch
       num += Om[(w * HD + dim) * OS + qr] * f;
       den += ml[w].y * f;
     }
-    op[(size_t)qrow * d + dim] = num / den;
+    if (p.op16)
+      put_plane(p.op16, row0 + qrow, hh * HD + dim, d / 32, num / den);
+    else
+      op[(size_t)qrow * d + dim] = num / den;
     if (p.lse && dim == 0)
       p.lse[fs.l + (size_t)qrow * H + hh] = mx * 0.69314718055994531f + logf(den);
   }
@@ -2519,12 +2936,16 @@ __device__ __forceinline__ bool flash_h3w_tile(const FlashParams& p, unsigned ch
   }
   if (__syncthreads_or(!finite)) return false;
   float* op = p.o + fs.o + hh * HD;
+  const int row0 = p.op16 ? (int)(fs.o / d) : 0;
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
     const int e = tid + i * 64 * NW;
     const int qr = e / HD, dim = e % HD, qrow = q0 + qr;
     if (qrow >= S) continue;
-    op[(size_t)qrow * d + dim] = res[i];
+    if (p.op16)
+      put_plane(p.op16, row0 + qrow, hh * HD + dim, d / 32, res[i]);
+    else
+      op[(size_t)qrow * d + dim] = res[i];
     if (p.lse && dim == 0) p.lse[fs.l + (size_t)qrow * H + hh] = lse[i];
   }
   return true;
@@ -2728,22 +3149,98 @@ hipError_t launch_gemm_x6(const GemmParams& p, int epi, hipStream_t s) {
   return hipGetLastError();
 }
 
+namespace {
+
+// Which kernel a split-fp16 GEMM runs, and the K ranges of its partial sums.
+enum H3Kind { H3_ROW1, H3_ROW2, H3_128K, H3_128, H3_256 };
+struct H3Plan {
+  H3Kind kind;
+  int splits;
+  int kc;  // k per split, whole steps of 32
+};
+
+// us on MI355X, weights from HBM: k1, k2 (k_gemm_h3k, 32 or 64 rows per
+// block), 128K (128 x 128 tiles, K dealt to two wave groups), 128 and 256
+// (256 x 128).
+H3Plan h3_plan(int M, int N, int K, bool parts) {
+  auto tiles = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+  // Splits while they fit one block per CU and leave each at least 192 k
+  // (768 x 768 at 64 rows: 7.7, 5.9, 5.2 us with 1, 2, 4).
+  auto splits = [&](long blocks) {
+    int n = 1;
+    while (parts && n < kGemmPartsMax && blocks * n * 2 <= 256 && K / (2 * n) >= 192) n *= 2;
+    return n;
+  };
+  auto plan = [&](H3Kind kind, int n) -> H3Plan {
+    const int kc = n > 1 ? ((K + n - 1) / n + 31) / 32 * 32 : K;
+    return {kind, (K + kc - 1) / kc, kc};
+  };
+  const long t128 = tiles(128, 128), t256 = tiles(256, 128), b1 = tiles(32, 64), b2 = tiles(64, 64);
+  // Fewer than about half a 128 x 128 tile per CU: short K chains win (870 x
+  // 2304 x 768, 126 tiles: k2 18.2, 128K 20.3; 870 x 3072 x 768, 168 tiles:
+  // 26.3 and 21.6).
+  if (t128 < 144) {
+    // One row tile per block while that still fits one block per CU at the
+    // split it needs (211 x 2304 x 768: k1 8.5, k2 9.2; 211 x 768 x 3072: 9.9
+    // in 2 splits, 9.2 in 4).
+    if (b1 <= 256 && (!parts || splits(b1) == splits(b2))) return plan(H3_ROW1, splits(b1));
+    return plan(H3_ROW2, splits(b2));
+  }
+  // 256 x 128 tiles where they fill most of every round of the CUs: 128 / 256,
+  // 8192 x 768 x 3072 (192 tiles, one round) 133 / 113, 8192 x 3072 x 768
+  // (768) 135 / 118, 2048 x 2304 x 768 (144) 34.9 / 33.4, but 8192 x 2304 x
+  // 768 (576, 2.25 rounds) 106.9 / 107.1 and 4096 x 2304 x 768 (288) 58 / 67.
+  if (t256 >= 1024 || (t256 > 128 && t256 <= 256) ||
+      (t256 > 256 && 10 * t256 >= 8 * 256 * ((t256 + 255) / 256)))
+    return plan(H3_256, 1);
+  // One 128 x 128 tile per CU at most: eight waves on each (4096 x 768 x
+  // 3072, 192 tiles: 128 80, 128K 66; 2048 x 2304 x 768, 288: 34.9 / 39.0).
+  return plan(t128 <= 256 ? H3_128K : H3_128, 1);
+}
+
+}  // namespace
+
+int gemm_h3_splits(int M, int N, int K) { return h3_plan(M, N, K, true).splits; }
+
 hipError_t launch_gemm_h3(const GemmParams& p, int epi, hipStream_t s) {
-  // K bounded so a block's rows (at most 256 of K floats) fit a buffer
-  // resource's 32-bit byte range.
-  if (p.K % 8 != 0 || p.M <= 0 || p.N <= 0 || p.K <= 0 || p.K > (1 << 20) || !p.a || !p.bp16 ||
-      !p.range_flag)
+  // K bounded so a block's planes (at most 256 rows of K) stay in a 32-bit
+  // byte range.
+  if (p.K % 8 != 0 || p.M <= 0 || p.N <= 0 || p.K <= 0 || p.K > (1 << 20) || !p.ap16 || !p.bp16 ||
+      !p.range_flag || (epi == GEMM_SILU && (!p.cp16 || p.N % 8 != 0)))
     return hipErrorInvalidValue;
-  // 256 x 128 tiles when there are at least four per CU, else 128 x 128
-  // (fewer idle CUs on the last round); measured on MI355X.
-  const bool big = (long)((p.M + 255) / 256) * ((p.N + 127) / 128) >= 1024;
-#define AKH_H3_GO(E)                                                                        \
-  if (big)                                                                                  \
-    hipLaunchKernelGGL((k_gemm_h3<E, 256, 128, 4, 2>),                                      \
-                       dim3((p.N + 127) / 128, (p.M + 255) / 256), dim3(512), 0, s, p);      \
-  else                                                                                      \
-    hipLaunchKernelGGL((k_gemm_h3<E, 128, 128, 2, 2>),                                      \
-                       dim3((p.N + 127) / 128, (p.M + 127) / 128), dim3(256), 0, s, p);
+  const bool parts = p.parts != nullptr;
+  if (parts && epi != GEMM_ADD) return hipErrorInvalidValue;
+  const H3Plan plan = h3_plan(p.M, p.N, p.K, parts);
+  GemmParams q = p;
+  q.split_kc = plan.kc;
+  if (plan.splits > 1) {  // partial sums: stored, not added
+    q.c = p.parts;
+    epi = GEMM_STORE;
+  }
+  const unsigned gz = (unsigned)plan.splits;
+#define AKH_H3_GO(E)                                                                          \
+  switch (plan.kind) {                                                                        \
+    case H3_ROW1:                                                                             \
+      hipLaunchKernelGGL((k_gemm_h3k<E, 1, 8, 4>), dim3((p.M + 31) / 32, (p.N + 63) / 64, gz), \
+                         dim3(512), 0, s, q);                                                 \
+      break;                                                                                  \
+    case H3_ROW2:                                                                             \
+      hipLaunchKernelGGL((k_gemm_h3k<E, 2, 8, 2>), dim3((p.M + 63) / 64, (p.N + 63) / 64, gz), \
+                         dim3(512), 0, s, q);                                                 \
+      break;                                                                                  \
+    case H3_128K:                                                                             \
+      hipLaunchKernelGGL((k_gemm_h3<E, 128, 128, 2, 2, 2, 2>),                                \
+                         dim3((p.N + 127) / 128, (p.M + 127) / 128, gz), dim3(512), 0, s, q); \
+      break;                                                                                  \
+    case H3_128:                                                                              \
+      hipLaunchKernelGGL((k_gemm_h3<E, 128, 128, 2, 2, 1, 2>),                                \
+                         dim3((p.N + 127) / 128, (p.M + 127) / 128), dim3(256), 0, s, q);     \
+      break;                                                                                  \
+    case H3_256:                                                                              \
+      hipLaunchKernelGGL((k_gemm_h3<E, 256, 128, 4, 2, 1, 3>),                                \
+                         dim3((p.N + 127) / 128, (p.M + 255) / 256), dim3(512), 0, s, q);     \
+      break;                                                                                  \
+  }
   switch (epi) {
     case GEMM_STORE: AKH_H3_GO(GEMM_STORE) break;
     case GEMM_ADD: AKH_H3_GO(GEMM_ADD) break;
@@ -2755,6 +3252,22 @@ hipError_t launch_gemm_h3(const GemmParams& p, int epi, hipStream_t s) {
   return hipGetLastError();
 }
 
+size_t split_rows_f16_bytes(size_t rows, int K) {
+  return (rows + 31) / 32 * ((K + 31) / 32) * 4096;
+}
+
+hipError_t launch_rows_planes(const float* x, int rows, int K, uint16_t* planes, hipStream_t s) {
+  if (rows <= 0 || K <= 0 || K % 8 != 0) return hipErrorInvalidValue;
+  const long n = (long)rows * ((K + 31) / 32) * 4;
+  hipLaunchKernelGGL(k_rows_planes, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, x, rows, K,
+                     planes);
+  return hipGetLastError();
+}
+
+size_t split_weights_f16_bytes(int K, int N) {
+  return (size_t)((N + 63) / 64) * ((K + 31) / 32) * 8192;
+}
+
 hipError_t launch_transpose_f32(const float* w, int K, int N, float* wt, hipStream_t s) {
   if (K <= 0 || N <= 0) return hipErrorInvalidValue;
   hipLaunchKernelGGL(k_transpose_f32, dim3((N + 31) / 32, (K + 31) / 32), dim3(256), 0, s, w, K,
@@ -2764,7 +3277,7 @@ hipError_t launch_transpose_f32(const float* w, int K, int N, float* wt, hipStre
 
 hipError_t launch_split_weights_f16(const float* w, int K, int N, uint16_t* wp, hipStream_t s) {
   if (K <= 0 || N <= 0 || K % 8 != 0) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_split_weights_f16, dim3((N + 31) / 32, (K + 31) / 32), dim3(256), 0, s, w,
+  hipLaunchKernelGGL(k_split_weights_f16, dim3((N + 63) / 64, (K + 31) / 32), dim3(256), 0, s, w,
                      K, N, wp);
   return hipGetLastError();
 }
@@ -2788,17 +3301,53 @@ hipError_t launch_flash_bf16(const FlashParams& p, int batch, int max_rows, hipS
   return hipGetLastError();
 }
 
-hipError_t launch_rows_rmsnorm(const float* x, const float* w, float* out,
-                               int rows, int size, float eps, hipStream_t s) {
+hipError_t launch_rows_rmsnorm(float* x, const float* w, float* out, int rows, int size,
+                               float eps, hipStream_t s, const float* parts, int nparts) {
   const dim3 g((rows + 3) / 4);
-  if (size % 4 != 0 || size > 4096)
-    hipLaunchKernelGGL(k_rows_rmsnorm<0>, dim3(rows), dim3(256), 0, s, x, w, out, rows, size, eps);
-  else if (size <= 1024)
-    hipLaunchKernelGGL(k_rows_rmsnorm<4>, g, dim3(256), 0, s, x, w, out, rows, size, eps);
-  else if (size <= 2048)
-    hipLaunchKernelGGL(k_rows_rmsnorm<8>, g, dim3(256), 0, s, x, w, out, rows, size, eps);
-  else
-    hipLaunchKernelGGL(k_rows_rmsnorm<16>, g, dim3(256), 0, s, x, w, out, rows, size, eps);
+  if (nparts > 0 && (!parts || size % 4 != 0 || size > kNormPartsMax)) return hipErrorInvalidValue;
+  if (nparts <= 0 && !out) return hipErrorInvalidValue;
+#define AKH_NORM_GO(QL)                                                                          \
+  if (nparts > 0)                                                                                \
+    hipLaunchKernelGGL((k_rows_rmsnorm<QL, true>), g, dim3(256), 0, s, x, w, out, rows, size,     \
+                       eps, parts, nparts);                                                      \
+  else                                                                                           \
+    hipLaunchKernelGGL((k_rows_rmsnorm<QL>), g, dim3(256), 0, s, x, w, out, rows, size, eps,      \
+                       nullptr, 0);
+  if (size % 4 != 0 || size > kNormPartsMax) {
+    hipLaunchKernelGGL(k_rows_rmsnorm<0>, dim3(rows), dim3(256), 0, s, x, w, out, rows, size, eps,
+                       nullptr, 0);
+  } else if (size <= 1024) {
+    AKH_NORM_GO(4)
+  } else if (size <= 2048) {
+    AKH_NORM_GO(8)
+  } else {
+    AKH_NORM_GO(16)
+  }
+#undef AKH_NORM_GO
+  return hipGetLastError();
+}
+
+hipError_t launch_rows_rmsnorm_planes(float* x, const float* w, uint16_t* planes, int rows,
+                                      int size, float eps, hipStream_t s, const float* parts,
+                                      int nparts) {
+  if (size % 8 != 0 || size > kNormPartsMax || rows <= 0 || !planes || (nparts > 0 && !parts))
+    return hipErrorInvalidValue;
+  const dim3 g((rows + 7) / 8);
+#define AKH_NORM_GO(QO)                                                                       \
+  if (nparts > 0)                                                                             \
+    hipLaunchKernelGGL((k_rows_rmsnorm_planes<QO, true>), g, dim3(512), 0, s, x, w, planes,    \
+                       rows, size, eps, parts, nparts);                                       \
+  else                                                                                        \
+    hipLaunchKernelGGL((k_rows_rmsnorm_planes<QO, false>), g, dim3(512), 0, s, x, w, planes,   \
+                       rows, size, eps, nullptr, 0);
+  if (size <= 1024) {
+    AKH_NORM_GO(2)
+  } else if (size <= 2048) {
+    AKH_NORM_GO(4)
+  } else {
+    AKH_NORM_GO(8)
+  }
+#undef AKH_NORM_GO
   return hipGetLastError();
 }
 

@@ -761,9 +761,12 @@ akh_status set_split(akh_model* m, int kind, bool fill) {
   for (uint32_t i = 0; i < m->packed.size(); ++i) {
     const PackedMatrix& pm = m->packed[i];
     if (!pm.rows) continue;
-    // Both copies take 4 bytes per element: an fp32 value, or two fp16 terms.
+    // Both copies take 4 bytes per element: an fp32 value, or two fp16 terms
+    // (padded to whole fragments).
     void* p = nullptr;
-    akh_status st = akh_tensor_alloc(m->be, (size_t)pm.K * pm.N * 4, &p);
+    akh_status st = akh_tensor_alloc(m->be, kind == AKH_SPLIT_H3
+                                                ? split_weights_f16_bytes(pm.K, pm.N)
+                                                : (size_t)pm.K * pm.N * 4, &p);
     if (st != AKH_OK) {
       set_split(m, AKH_SPLIT_NONE, false);
       return st;
@@ -1162,6 +1165,8 @@ struct akh_session {
   // Prefill buffers, grown on demand to the prompt rows (B * prompt_len, or
   // the sum of ragged prompt lengths).
   size_t prows = 0;
+  float* pparts = nullptr;  // partial sums of the prefill's few-row GEMMs
+  float* pwide = nullptr;   // fp32 normed rows wider than kNormPartsMax
   float *px = nullptr, *pxn = nullptr, *pq = nullptr, *pattn = nullptr,
         *pffn = nullptr;
   uint32_t* ptok = nullptr;
@@ -1216,12 +1221,14 @@ int lm_parts_max(const akh_session* s) {
 int argmax_parts(const akh_session* s) { return s->generic ? 1 : lm_parts(s); }
 
 void free_prefill(akh_session* s) {
-  for (float* p : {s->px, s->pxn, s->pq, s->pattn, s->pffn, s->pk, s->pv})
+  for (float* p : {s->px, s->pxn, s->pq, s->pattn, s->pffn, s->pk, s->pv, s->pparts,
+                   s->pwide})
     if (p) hipFree(p);
   for (void* p : {(void*)s->ptok, (void*)s->p_at, (void*)s->p_map, (void*)s->p_last,
                   (void*)s->p_len})
     if (p) hipFree(p);
-  s->px = s->pxn = s->pq = s->pattn = s->pffn = s->pk = s->pv = nullptr;
+  s->px = s->pxn = s->pq = s->pattn = s->pffn = s->pk = s->pv = s->pparts = s->pwide =
+      nullptr;
   s->ptok = nullptr;
   s->p_at = s->p_last = s->p_len = nullptr;
   s->p_map = nullptr;
@@ -1233,10 +1240,14 @@ akh_status ensure_prefill(akh_session* s, size_t rows) {
   free_prefill(s);
   const size_t d = s->m->cfg.dim, F = s->m->cfg.ffn_hidden;
   HIP_TRY(hipMalloc(&s->px, rows * d * 4));
-  HIP_TRY(hipMalloc(&s->pxn, rows * d * 4));
+  // The GEMMs' A operands: fp32 rows, or the same rows' fp16 planes (padded to
+  // whole fragments).
+  HIP_TRY(hipMalloc(&s->pxn, split_rows_f16_bytes(rows, (int)d)));
   HIP_TRY(hipMalloc(&s->pq, rows * d * 4));
-  HIP_TRY(hipMalloc(&s->pattn, rows * d * 4));
-  HIP_TRY(hipMalloc(&s->pffn, rows * F * 4));
+  HIP_TRY(hipMalloc(&s->pattn, split_rows_f16_bytes(rows, (int)d)));
+  HIP_TRY(hipMalloc(&s->pffn, split_rows_f16_bytes(rows, (int)F)));
+  HIP_TRY(hipMalloc(&s->pparts, kGemmPartsFloats * 4));
+  if (d > (size_t)kNormPartsMax) HIP_TRY(hipMalloc(&s->pwide, rows * d * 4));
   HIP_TRY(hipMalloc(&s->ptok, rows * 4));
   HIP_TRY(hipMalloc(&s->p_at, (s->B + 1) * sizeof(int)));
   HIP_TRY(hipMalloc(&s->p_map, rows * sizeof(int2)));
@@ -1879,7 +1890,8 @@ extern "C" akh_status akh_session_truncate(akh_session* s, uint32_t len) {
 namespace {
 
 // A prefill GEMM on parameter `index`: the model's split kernel on its copy
-// of the matrix, or the fp32-MFMA kernel (no copy, or `exact`).
+// of the matrix (split-fp16: A from g.ap16's planes), or the fp32-MFMA kernel
+// (no copy, or `exact`).
 hipError_t prefill_gemm(const akh_model* m, GemmParams& g, uint32_t index, int epi,
                         hipStream_t st, bool exact) {
   if (!exact && index < m->wsplit.size() && m->wsplit[index]) {
@@ -1922,6 +1934,24 @@ struct PrefillRows {
   bool ragged = false;
 };
 
+// The RMSNorm of px into pxn, as fp32 rows or the fp16 planes of the
+// split-fp16 GEMMs' A, after adding the `pending` partial sums px still lacks.
+hipError_t prefill_norm(akh_session* s, const float* gain, size_t rows, bool planes,
+                        int pending) {
+  const int d = (int)s->m->cfg.dim;
+  const float eps = s->m->cfg.norm_eps;
+  hipStream_t st = s->be->stream;
+  uint16_t* xn16 = reinterpret_cast<uint16_t*>(s->pxn);
+  if (planes && d <= kNormPartsMax)
+    return launch_rows_rmsnorm_planes(s->px, gain, xn16, (int)rows, d, eps, st, s->pparts,
+                                      pending);
+  if (!planes)
+    return launch_rows_rmsnorm(s->px, gain, s->pxn, (int)rows, d, eps, st, s->pparts, pending);
+  // Rows wider than the norm's registers: fp32 rows first.
+  hipError_t e = launch_rows_rmsnorm(s->px, gain, s->pwide, (int)rows, d, eps, st);
+  return e == hipSuccess ? launch_rows_planes(s->pwide, (int)rows, d, xn16, st) : e;
+}
+
 // The prefill layers in fp32 (build_prefill_layer's node order); `exact`
 // runs them on the fp32-MFMA kernels whatever the model's split kernels.
 hipError_t prefill_layers_f32(akh_session* s, const PrefillRows& pr, bool exact) {
@@ -1934,11 +1964,30 @@ hipError_t prefill_layers_f32(akh_session* s, const PrefillRows& pr, bool exact)
     const hipError_t e_ = (x);          \
     if (e_ != hipSuccess) return e_;    \
   } while (0)
+  // On the split-fp16 kernels every GEMM's A is written as fp16 planes by the
+  // kernel before it (norm, flash, ffn_up's SiLU), and out_proj and ffn_down
+  // on few rows leave the partial sums of several K ranges for the norm after
+  // them to add to px.
+  const bool h3 = !exact && h3_prefill(s->m);
+  const bool parts = h3 && d <= (uint32_t)kNormPartsMax;
+  uint16_t* xn16 = reinterpret_cast<uint16_t*>(s->pxn);
+  uint16_t* attn16 = reinterpret_cast<uint16_t*>(s->pattn);
+  uint16_t* ffn16 = reinterpret_cast<uint16_t*>(s->pffn);
+  int pending = 0;  // partial sums px still lacks
+  auto add_gemm = [&](GemmParams& g, uint32_t index) -> hipError_t {
+    g.parts = parts ? s->pparts : nullptr;
+    const int n = parts ? gemm_h3_splits(g.M, g.N, g.K) : 1;
+    pending = n > 1 ? n : 0;
+    return prefill_gemm(s->m, g, index, GEMM_ADD, st, exact);
+  };
+  auto norm = [&](uint32_t l, int which) -> hipError_t {
+    return prefill_norm(s, s->m->layer(l, which), rows, h3, pending);
+  };
   for (uint32_t l = 0; l < c.num_layers; ++l) {
-    TRY_HIP(launch_rows_rmsnorm(s->px, s->m->layer(l, W_NORM1), s->pxn,
-                                (int)rows, (int)d, c.norm_eps, st));
+    TRY_HIP(norm(l, W_NORM1));
     GemmParams g{};
     g.a = s->pxn;
+    g.ap16 = xn16;
     g.b = s->m->layer(l, W_QKV);
     g.M = (int)rows;
     g.N = 3 * d;
@@ -1981,23 +2030,29 @@ hipError_t prefill_layers_f32(akh_session* s, const PrefillRows& pr, bool exact)
            : s->m->prefill_split == AKH_SPLIT_H3          ? FLASH_H3
                                                           : FLASH_X6;
     f.range_flag = s->m->range_flag;
-    TRY_HIP(launch_flash(f, (int)s->B, (int)S, st));
-
     GemmParams o{};
     o.a = s->pattn;
+    o.ap16 = attn16;
+    if (h3 && flash_writes_planes(f)) f.op16 = attn16;
+    TRY_HIP(launch_flash(f, (int)s->B, (int)S, st));
+    if (h3 && !f.op16) {  // the other head sizes' fp32 rows (xn is free)
+      TRY_HIP(launch_rows_planes(s->pattn, (int)rows, (int)d, xn16, st));
+      o.ap16 = xn16;
+    }
     o.b = s->m->layer(l, W_OUT);
     o.c = s->px;
     o.M = (int)rows;
     o.N = d;
     o.K = d;
-    TRY_HIP(prefill_gemm(s->m, o, base + W_OUT, GEMM_ADD, st, exact));
+    TRY_HIP(add_gemm(o, base + W_OUT));
 
-    TRY_HIP(launch_rows_rmsnorm(s->px, s->m->layer(l, W_NORM2), s->pxn,
-                                (int)rows, (int)d, c.norm_eps, st));
+    TRY_HIP(norm(l, W_NORM2));
     GemmParams u{};
     u.a = s->pxn;
+    u.ap16 = xn16;
     u.b = s->m->layer(l, W_UP);
     u.c = s->pffn;
+    u.cp16 = ffn16;
     u.M = (int)rows;
     u.N = c.ffn_hidden;
     u.K = d;
@@ -2005,13 +2060,17 @@ hipError_t prefill_layers_f32(akh_session* s, const PrefillRows& pr, bool exact)
 
     GemmParams w{};
     w.a = s->pffn;
+    w.ap16 = ffn16;
     w.b = s->m->layer(l, W_DOWN);
     w.c = s->px;
     w.M = (int)rows;
     w.N = d;
     w.K = c.ffn_hidden;
-    TRY_HIP(prefill_gemm(s->m, w, base + W_DOWN, GEMM_ADD, st, exact));
+    TRY_HIP(add_gemm(w, base + W_DOWN));
   }
+  if (pending > 0)  // the last ffn_down's, with no norm: px alone
+    TRY_HIP(launch_rows_rmsnorm(s->px, nullptr, nullptr, (int)rows, (int)d, c.norm_eps, st,
+                                s->pparts, pending));
 #undef TRY_HIP
   return hipSuccess;
 }
@@ -2816,11 +2875,10 @@ extern "C" akh_status akh_forward_loss(akh_forward* f, const uint32_t* tokens,
                                          V, st);
     if (e == hipSuccess)
       e = f->m->prefill_bf16 ? prefill_layers_bf16(s, pr) : prefill_layers_f32(s, pr, exact);
-    if (e == hipSuccess)
-      e = launch_rows_rmsnorm(s->px, f->m->final_norm(), s->pxn, (int)rows, (int)d, c.norm_eps,
-                              st);
+    if (e == hipSuccess) e = prefill_norm(s, f->m->final_norm(), rows, h3 && !exact, 0);
     GemmParams g{};
     g.a = s->pxn;
+    g.ap16 = reinterpret_cast<const uint16_t*>(s->pxn);
     g.b = f->m->lm_head();
     g.c = f->logits;
     g.M = (int)rows;

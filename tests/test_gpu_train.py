@@ -10,6 +10,8 @@ stream to 1e-3 (train.rs:928-945); elementwise shaders are exact or within
 an ulp of libm.
 """
 
+import dataclasses
+
 import numpy as np
 import pytest
 
@@ -206,4 +208,37 @@ def test_forward_x6_ragged_k(backend, pkg, ora):
     np.testing.assert_allclose(losses, ol, atol=1e-4)
     np.testing.assert_allclose(f.hidden(), oh, atol=1e-4)
     np.testing.assert_allclose(f.probs(0, 22), op, atol=1e-5)
+    f.close()
+
+
+# The split-fp16 GEMMs' kernels by grid: rows of one and of two 32-row tiles per
+# block with K dealt to the waves (one row, a partial second tile, K ranges
+# whose partial sums the next norm adds), 128 x 128 tiles by two wave groups
+# (an odd number of K steps: one group sits out the last) and by one, and 256 x
+# 128; ffn 200, 1000 and 2088 leave K steps and column groups partly empty.
+@pytest.mark.parametrize("batch,seq,dim,ffn", [
+    (1, 1, 64, 200), (1, 33, 64, 1000), (3, 45, 128, 2088), (2, 150, 64, 4096),
+    (5, 61, 192, 8192), (4, 275, 96, 2088), (9, 256, 64, 4104), (5, 256, 128, 3328),
+])
+def test_forward_h3_grids_match_fp32_mfma(backend, pkg, batch, seq, dim, ffn):
+    M = pkg.hip.Model
+    cfg = dataclasses.replace(pkg.ModelConfig.new(97, dim, dim // (32 if dim == 96 else 64), 2, seq),
+                              ffn_hidden=ffn)
+    model = M(backend, cfg)
+    model.upload(pkg.synthetic_weights(cfg, seed=67))
+    assert model.prefill_split() == M.SPLIT_H3
+    toks = pkg.synthetic_tokens(batch * seq, 97, seed=68)
+    tgts = pkg.synthetic_tokens(batch * seq, 97, seed=69)
+    f = pkg.hip.Forward(model, batch, seq)
+    _, lh = f.loss(toks, tgts)
+    hh = f.hidden()
+    _, again = f.loss(toks, tgts)
+    assert np.array_equal(lh, again)
+    model.set_prefill_split(M.SPLIT_NONE)
+    _, lf = f.loss(toks, tgts)
+    # Either kernel is off by at most (2^-22 + sqrt(K) 2^-24) sum |a b| per
+    # product row, with sum |a b| below 4 and K up to 8192 here.
+    tol = 2 * 4 * (2.0 ** -22 + np.sqrt(max(dim, ffn)) * 2.0 ** -24)
+    assert np.abs(hh - f.hidden()).max() < 2 * tol  # two layers
+    assert np.abs(lh - lf).max() < 4 * tol  # the lm_head on rows scaled by the norm
     f.close()
