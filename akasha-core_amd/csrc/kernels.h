@@ -196,9 +196,9 @@ hipError_t launch_gemm_x6(const GemmParams& p, int epi, hipStream_t s);
 // operand beyond fp16's range); the caller then recomputes in fp32.  K % 8 == 0.
 hipError_t launch_gemm_h3(const GemmParams& p, int epi, hipStream_t s);
 // K ranges whose partial sums launch_gemm_h3 stores to p.parts (1: none).
-// They take at most one 64 x 64 tile per CU and split.
+// They take at most one 128 x 128 tile per CU.
 constexpr int kGemmPartsMax = 8;
-constexpr size_t kGemmPartsFloats = 256 * 64 * 64;
+constexpr size_t kGemmPartsFloats = 256 * 128 * 128;
 int gemm_h3_splits(int M, int N, int K);
 // The fp16 planes of a [K, N] row-major matrix for launch_gemm_h3.
 size_t split_weights_f16_bytes(int K, int N);

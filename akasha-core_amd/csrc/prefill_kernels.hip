@@ -3176,6 +3176,14 @@ H3Plan h3_plan(int M, int N, int K, bool parts) {
     return {kind, (K + kc - 1) / kc, kc};
   };
   const long t128 = tiles(128, 128), t256 = tiles(256, 128), b1 = tiles(32, 64), b2 = tiles(64, 64);
+  // Partial sums of 128 x 128 tiles that fill the CUs in two to four K ranges
+  // (2048 x 768 x 3072, 96 tiles: k2 65, 128K 55, in 2 ranges 34; 400 x 2048 x
+  // 8192, 64 tiles: 62, 153, in 4 ranges 53; 911 x 768 x 3072, 48 tiles: k2
+  // 23.5, in 4 ranges 21.2 before the norm reads four parts instead of none).
+  if (parts && t128 >= 56 && t128 <= 128) {
+    const int n = (int)(256 / t128);
+    if (K / n >= 768) return plan(H3_128K, n);
+  }
   // Fewer than about half a 128 x 128 tile per CU: short K chains win (870 x
   // 2304 x 768, 126 tiles: k2 18.2, 128K 20.3; 870 x 3072 x 768, 168 tiles:
   // 26.3 and 21.6).

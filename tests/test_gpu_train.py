@@ -214,11 +214,13 @@ def test_forward_x6_ragged_k(backend, pkg, ora):
 # The split-fp16 GEMMs' kernels by grid: rows of one and of two 32-row tiles per
 # block with K dealt to the waves (one row, a partial second tile, K ranges
 # whose partial sums the next norm adds), 128 x 128 tiles by two wave groups
-# (an odd number of K steps: one group sits out the last) and by one, and 256 x
-# 128; ffn 200, 1000 and 2088 leave K steps and column groups partly empty.
+# (an odd number of K steps: one group sits out the last; whole or in K ranges)
+# and by one, and 256 x 128; ffn 200, 1000 and 2088 leave K steps and column
+# groups partly empty.
 @pytest.mark.parametrize("batch,seq,dim,ffn", [
     (1, 1, 64, 200), (1, 33, 64, 1000), (3, 45, 128, 2088), (2, 150, 64, 4096),
     (5, 61, 192, 8192), (4, 275, 96, 2088), (9, 256, 64, 4104), (5, 256, 128, 3328),
+    (8, 450, 256, 3080),
 ])
 def test_forward_h3_grids_match_fp32_mfma(backend, pkg, batch, seq, dim, ffn):
     M = pkg.hip.Model
