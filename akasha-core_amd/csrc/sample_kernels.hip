@@ -1,5 +1,5 @@
 // Device-side token choice: sample_token of src/nn/sampling.rs:3-81 for a
-// batch of rows, one 1024-thread block per row (or per part of a row, below).
+// batch of rows, one 1024-thread block per row.
 //
 // The reference copies the logits, applies the repetition penalty to every
 // distinct seen id, and then either takes the argmax (temperature <= 0) or
@@ -20,17 +20,19 @@
 // scratch row; the repetition penalty is applied on the fly through a bitmap
 // of the seen ids in LDS.
 //
-// With 0 < top_k <= 1024 (run_chat's 40) only the top_k elements matter:
-// a cut on d = max - l admitting between top_k and 2048 elements is found
-// by counting against 16 thresholds per pass (powers of four, then 16-way
-// refinements), those elements are gathered to LDS and each takes its place
-// in the order (logit descending, index ascending) by counting the entries
-// above it; the first top_k then go through the reference's own sequence:
-// f64 probabilities summed in order, the top_p prefix, the walk r -= p.
-// With top_k <= 256 a row is split over several blocks (parts of the
-// vocabulary), whose top_k the row's last block merges.  NaN or infinite
-// maxima, fewer than top_k finite elements and ties too wide for the cut
-// take the radix path.
+// Rows of at least kHistMin ids skip that: a first kernel spreads each row
+// over several blocks, which bin their part's logits on a fixed grid (2047
+// bins below the part's maximum) and sum each bin's f64 weights, or count its
+// elements where 0 < top_k <= 1024.  The row's block adds the parts' bins,
+// finds the bins in which the cuts fall, gathers their members (a few hundred
+// ids), puts them in order by counting the entries above each, and cuts
+// exactly there.  With top_k that list is the top_k, which then goes through
+// the reference's own sequence: f64 probabilities summed in order, the top_p
+// prefix, the walk r -= p.  NaN, an infinite maximum, cuts below the bins and
+// bins of too many ids (ties) take the radix path.
+// Shorter rows with 0 < top_k <= 1024: a cut on d = max - l admitting between
+// top_k and 2048 elements is found by counting against 16 thresholds per pass
+// (powers of four, then 16-way refinements) instead of the bins.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -49,7 +51,7 @@ namespace {
 #ifndef AKH_SAMPLE_BLOCKS
 #define AKH_SAMPLE_BLOCKS 256
 #endif
-constexpr int NT = AKH_SAMPLE_NT;  // threads per row (per part of a split row)
+constexpr int NT = AKH_SAMPLE_NT;  // threads per row (per part of a binned row)
 constexpr int NW = NT / 64;     // waves per block
 
 // Radix digits of the order keys: 11, 11 and 10 bits (three passes).
@@ -248,8 +250,13 @@ constexpr int NTH = 16;     // thresholds counted per pass
 
 struct TopKShared {
   unsigned long long comp[CCAP];  // key << 32 | ~index: descending = the order
-  unsigned long long top[KCAP];   // the first entries of that order
-  double prob[KCAP];
+  union {
+    struct {
+      unsigned long long top[KCAP];  // the first entries of that order
+      double prob[KCAP];
+    };
+    unsigned long long sorted[CCAP];  // all of them
+  };
   double norm;
   int keep;
   uint32_t wcnt[NW][NTH];
@@ -278,6 +285,18 @@ __device__ __forceinline__ int rank_top(int nc, int K, TopKShared& tk) {
   }
   __syncthreads();
   return min(nc, K);
+}
+
+// The same for every entry, into tk.sorted.
+__device__ __forceinline__ void rank_all(int nc, TopKShared& tk) {
+  for (int e = threadIdx.x; e < nc; e += NT) {
+    const unsigned long long x = tk.comp[e];
+    int above = 0;
+#pragma unroll 8
+    for (int f = 0; f < nc; ++f) above += tk.comp[f] > x ? 1 : 0;
+    tk.sorted[above] = x;
+  }
+  __syncthreads();
 }
 
 // sampling.rs:45-80 over tk.top[0 .. top_k) in the reference's order: f64
@@ -381,20 +400,40 @@ __device__ void reduce_counts(const uint32_t (&c)[NTH], uint32_t base, TopKShare
   __syncthreads();
 }
 
-// The top_k elements of l_of(0 .. n) (0 < top_k <= KCAP) in order in
-// tk.top (index idx0 + i), from at most CCAP candidates gathered to tk.comp:
-// returns how many (top_k, or fewer with all_finite), or -1 where the radix path must decide instead
-// (NaN, an infinite maximum, fewer than top_k finite elements near the
-// maximum, ties too wide to cut).  With all_finite, fewer than top_k finite
-// elements near the maximum gathers every finite element instead (a part
-// of a row, which may hold fewer than top_k).  Every thread of the block
-// calls it; the outcome is the same for all.  The first count bins d =
+// tk.comp[0 .. tk.n_cand) = the elements of the row that `take` accepts, in
+// any order (n_cand counts those past CCAP too).
+template <typename LFn, typename TakeFn>
+__device__ __forceinline__ void gather(int n, LFn l_of, TakeFn take, TopKShared& tk) {
+  if (threadIdx.x == 0) tk.n_cand = 0;
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  for_row(n, l_of, [&](float l, int i, bool live) {
+    const bool in = live && take(l);
+    const unsigned long long mask = __ballot(in);
+    if (mask) {
+      const int lead = __ffsll((long long)mask) - 1;
+      uint32_t base = 0;
+      if (lane == lead) base = atomicAdd(&tk.n_cand, (uint32_t)__popcll(mask));
+      base = __shfl(base, lead, 64);
+      const uint32_t slot = base + __popcll(mask & ((1ull << lane) - 1ull));
+      if (in && slot < (uint32_t)CCAP)
+        tk.comp[slot] = ((unsigned long long)order_key(l) << 32) | (0xFFFFFFFFu - (uint32_t)i);
+    }
+  });
+  __syncthreads();
+}
+
+// The top_k elements of l_of(0 .. n) (0 < top_k <= KCAP) in order in tk.top,
+// from at most CCAP candidates gathered to tk.comp: returns how many, or -1
+// where the radix path must decide instead (NaN, an infinite maximum, fewer
+// than top_k finite elements near the maximum, ties too wide to cut).  Every
+// thread of the block calls it; the outcome is the same for all.  The first count bins d =
 // max - l by its binary exponent (d < 2^(2j - 12) exactly when its
 // exponent is below 2j - 12), four packed 8-bit counters per chunk;
 // refinements compare only the elements inside the narrowed interval.
 template <typename LFn>
-__device__ __forceinline__ int topk_candidates(int n, LFn l_of, uint32_t idx0, uint32_t top_k,
-                                              bool all_finite, SampleShared& sh, TopKShared& tk) {
+__device__ __forceinline__ int topk_candidates(int n, LFn l_of, uint32_t top_k,
+                                               SampleShared& sh, TopKShared& tk) {
   float mxv = -INFINITY;
   uint32_t nan = 0;
   for_row(n, l_of, [&](float l, int, bool) {
@@ -403,7 +442,6 @@ __device__ __forceinline__ int topk_candidates(int n, LFn l_of, uint32_t idx0, u
   });
   const float mx = block_max_f(mxv, sh);
   if (block_sum_u(nan, sh) != 0) return -1;
-  if (mx == -INFINITY && all_finite) return 0;  // a part with no finite element
   if (!isfinite(mx)) return -1;
 
   // Threshold t: 2^(2t - 12) in the first count, then (lo, hi] cut in NTH.
@@ -445,11 +483,7 @@ __device__ __forceinline__ int topk_candidates(int n, LFn l_of, uint32_t idx0, u
   for (int round = 0; round < 4; ++round) {
     int j = 0;
     while (j < NTH && tk.cnt[j] < top_k) ++j;
-    if (j == NTH) {  // fewer than top_k finite elements near the max
-      if (!all_finite) return -1;
-      cut = INFINITY;
-      break;
-    }
+    if (j == NTH) return -1;  // fewer than top_k finite elements near the max
     if (tk.cnt[j] <= (uint32_t)(round == 0 ? CCAP / 4 : CCAP)) {
       cut = thr(j);
       break;
@@ -477,180 +511,354 @@ __device__ __forceinline__ int topk_candidates(int n, LFn l_of, uint32_t idx0, u
     reduce_counts(c, base, tk);
   }
 
-  // Gather the elements under the cut.
-  if (threadIdx.x == 0) tk.n_cand = 0;
-  __syncthreads();
-  const int lane = threadIdx.x & 63;
-  for_row(n, l_of, [&](float l, int i, bool live) {
-    const bool take = live && mx - l < cut;
-    const unsigned long long mask = __ballot(take);
-    if (mask) {
-      const int lead = __ffsll((long long)mask) - 1;
-      uint32_t base = 0;
-      if (lane == lead) base = atomicAdd(&tk.n_cand, (uint32_t)__popcll(mask));
-      base = __shfl(base, lead, 64);
-      const uint32_t slot = base + __popcll(mask & ((1ull << lane) - 1ull));
-      if (take && slot < (uint32_t)CCAP)
-        tk.comp[slot] = ((unsigned long long)order_key(l) << 32) | (0xFFFFFFFFu - (idx0 + (uint32_t)i));
-    }
-  });
-  __syncthreads();
+  gather(n, l_of, [&](float l) { return mx - l < cut; }, tk);
   const int nc = (int)tk.n_cand;
-  if (nc > CCAP || (!all_finite && nc < (int)top_k)) return -1;
+  if (nc > CCAP || nc < (int)top_k) return -1;
   return rank_top(nc, (int)top_k, tk);
 }
 
-__global__ __launch_bounds__(NT) void k_sample_rows(SampleArgs a) {
+// This row's seen ids (positions [lo, hi) of ids, a row of len entries).
+struct SeenIds {
+  const uint32_t* ids = nullptr;
+  long len = 0;
+  int lo = 0, hi = 0;
+};
+
+// The bitmap of a row's seen ids (null if the penalty changes nothing).  The
+// ids are read from their whole row (its extent is known) while the range is
+// still being loaded.
+__device__ __forceinline__ const uint32_t* seen_bitmap(const SampleArgs& a, const SeenIds& s,
+                                                       uint32_t* bitmap) {
+  if (a.penalty == 1.0f || !s.ids) return nullptr;
+  const int words = (a.n + 31) / 32;
+  for (long s0 = 0; s0 < s.len; s0 += 4 * NT) {
+    uint32_t v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const long q = s0 + u * NT + threadIdx.x;
+      v[u] = q < s.len ? s.ids[q] : 0u;
+    }
+    if (s0 == 0) {
+      for (int k = threadIdx.x; k < words; k += NT) bitmap[k] = 0;
+      __syncthreads();
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const long q = s0 + u * NT + threadIdx.x;
+      if (q >= s.lo && q < s.hi && v[u] < (uint32_t)a.n)
+        atomicOr(&bitmap[v[u] >> 5], 1u << (v[u] & 31));
+    }
+  }
+  if (s.len <= 0) {
+    for (int k = threadIdx.x; k < words; k += NT) bitmap[k] = 0;
+  }
+  __syncthreads();
+  return bitmap;
+}
+
+// Row m's seen ids; false if the row is done (session mode).
+__device__ __forceinline__ bool row_seen(const SampleArgs& a, int m, SeenIds& s) {
+  if (a.tok) {
+    const int dn = a.done[m], st = a.start[m], p = a.pos[m];
+    if (dn) return false;
+    s.ids = a.hist + (size_t)m * a.hist_stride;
+    s.len = a.hist_stride;
+    s.lo = st;
+    s.hi = p > st ? p : st;
+  } else if (a.seen) {
+    s.ids = a.seen + (size_t)m * a.seen_stride;
+    s.len = a.seen_stride;
+    s.hi = a.seen_len ? (int)min(a.seen_len[m], (uint32_t)a.seen_stride) : 0;
+  }
+  return true;
+}
+
+// ---------------------------------------------------------------------------
+// Binned rows.  Logit l lies in grid cell floor(l * scale); the bins of a part
+// (and of the row) are the kCells cells from its maximum's down, bin d the
+// cell d below.  What lies further below is only in the part's total.  The
+// row's workspace holds kBins doubles per part (f64 weights relative to the
+// part's maximum, or uint32 counts), then a header per part.
+// ---------------------------------------------------------------------------
+constexpr int kCells = kBins - 1;
+constexpr int kPartsMax = 16;
+struct PartHead {
+  float max;
+  int bad;       // NaN, an infinite maximum, a grid beyond 2^30
+  double total;  // of the part's weights (or its count)
+};
+static_assert(sizeof(PartHead) == 2 * sizeof(double), "two doubles of the row's workspace");
+static_assert(kBins == 2 * NT && CCAP == 2 * NT, "two bins and two list entries per thread");
+constexpr int kHistMin = kBins + 2;  // ids: one part's bins and header
+
+// About 64 cells per logit or 48 per unit of l / T, whichever is finer: cells
+// of ~150 ids at the densest of 50257 logits N(0, 2^2), and 2047 cells reach
+// 42 T below the maximum (e^-42 of its weight) or 32.
+__device__ __forceinline__ float grid_scale(float temperature) {
+  return fmaxf(64.0f, 48.0f / temperature);
+}
+__device__ __forceinline__ float grid_cell(float l, float scale) {
+  return floorf(__fmul_rn(l, scale));
+}
+
+__global__ __launch_bounds__(NT) void k_sample_hist(SampleArgs a) {
+  extern __shared__ uint32_t bitmap[];
+  __shared__ SampleShared sh;
+  const int m = blockIdx.x, part = blockIdx.y, parts = gridDim.y;
+  SeenIds seen;
+  if (!row_seen(a, m, seen)) return;
+  const uint32_t* bm = seen_bitmap(a, seen, bitmap);
+  const bool count = a.top_k > 0 && a.top_k < a.n;
+  const float* row = a.logits + (size_t)m * a.row_stride;
+  const int per = (a.n + parts - 1) / parts, lo = min(a.n, part * per);
+  const int len = min(a.n, lo + per) - lo;
+  auto l_at = [&](int i) { return pen_logit(row, lo + i, bm, a.penalty); };
+  // A part of up to NT * U ids stays in registers between the two passes.
+  float v[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int i = u * NT + (int)threadIdx.x;
+    v[u] = i < len ? l_at(i) : -INFINITY;
+  }
+  auto each = [&](auto f) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) f(v[u]);
+    for (int i = U * NT + (int)threadIdx.x; i < len; i += NT) f(l_at(i));
+  };
+  float mxv = -INFINITY;
+  uint32_t nan = 0;
+  each([&](float l) {
+    if (l != l) nan = 1;
+    else mxv = fmaxf(mxv, l);
+  });
+  for (int b = threadIdx.x; b < kBins; b += NT) {
+    if (count) sh.hist_n[b] = 0u;
+    else sh.hist_w[b] = 0.0;
+  }
+  const float mx = block_max_f(mxv, sh);
+  const float scale = grid_scale(a.temperature);
+  const bool empty = mx == -INFINITY;
+  const bool bad = block_sum_u(nan, sh) != 0 || mx == INFINITY ||
+                   (!empty && !(fabsf(mx) * scale < 0x1p30f));
+  double own = 0.0;
+  if (!bad && !empty) {
+    const float cell = grid_cell(mx, scale);
+    const double mxd = (double)mx, T = (double)a.temperature;
+    each([&](float l) {
+      const float d = cell - grid_cell(l, scale);
+      const bool in = d < (float)kCells;
+      if (count) {
+        if (in) atomicAdd(&sh.hist_n[(int)d], 1u);
+      } else if (l > -INFINITY) {
+        const double w = exp(((double)l - mxd) / T);
+        own += w;
+        if (in) atomicAdd(&sh.hist_w[(int)d], w);
+      }
+    });
+  }
+  const double total = block_sum_d(own, sh);  // its barriers complete the bins
+  double* base = a.wbuf + (size_t)m * a.n;
+  if (!bad && !empty) {
+    double* bins = base + (size_t)part * kBins;
+    for (int b = threadIdx.x; b < kBins; b += NT) {
+      if (count) reinterpret_cast<uint32_t*>(bins)[b] = sh.hist_n[b];
+      else bins[b] = sh.hist_w[b];
+    }
+  }
+  if (threadIdx.x == 0)
+    reinterpret_cast<PartHead*>(base + (size_t)parts * kBins)[part] = PartHead{mx, bad, total};
+}
+
+struct RowHist {
+  double before[kBins];  // weight (or count) of the bins above
+  float part_max[kPartsMax];
+  double part_f[kPartsMax];
+  uint32_t first[8];     // list position of a bin's first entry
+  double pre[CCAP];      // weight of the list's entries before each
+  double target;
+  uint32_t lo, hi, cut;
+};
+
+// The pick of row m from its parts' bins, or n where the radix path must
+// decide.  Every thread of the block calls it.
+template <typename LFn>
+__device__ __forceinline__ uint32_t pick_binned(const SampleArgs& a, int m, int parts, LFn l_of,
+                                                double r, SampleShared& sh, TopKShared& tk,
+                                                RowHist& rh) {
+  const uint32_t none = (uint32_t)a.n;
+  const int n = a.n, t = threadIdx.x;
+  const bool count = a.top_k > 0 && a.top_k < n;
+  const float scale = grid_scale(a.temperature);
+  const double* base = a.wbuf + (size_t)m * n;
+  const PartHead* head = reinterpret_cast<const PartHead*>(base + (size_t)parts * kBins);
+  float mx = -INFINITY;
+  int bad = 0;
+  for (int q = 0; q < parts; ++q) {
+    mx = fmaxf(mx, head[q].max);
+    bad |= head[q].bad;
+  }
+  if (bad || mx == -INFINITY) return none;  // uniform
+  const double mxd = (double)mx, T = (double)a.temperature;
+  if (t < parts) {
+    rh.part_max[t] = head[t].max;
+    rh.part_f[t] = head[t].max == -INFINITY ? 0.0 : exp(((double)head[t].max - mxd) / T);
+  }
+  __syncthreads();
+  double total = 0.0;
+  for (int q = 0; q < parts; ++q) total += rh.part_f[q] * head[q].total;
+
+  // Thread t's bins 2 t and 2 t + 1 over the parts, then every bin's total
+  // above it.
+  const float cell = grid_cell(mx, scale);
+  double v[2] = {0.0, 0.0};
+  for (int q = 0; q < parts; ++q) {
+    const float off = cell - grid_cell(rh.part_max[q], scale);  // inf: an empty part
+    if (!(off < (float)kCells)) continue;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int b = 2 * t + e - (int)off;
+      if (b < 0 || 2 * t + e >= kCells) continue;
+      v[e] += count ? (double)reinterpret_cast<const uint32_t*>(base + (size_t)q * kBins)[b]
+                    : rh.part_f[q] * base[(size_t)q * kBins + b];
+    }
+  }
+  const double above = block_scan_excl<double>(v[0] + v[1], sh.wave_d);
+  rh.before[2 * t] = above;
+  rh.before[2 * t + 1] = above + v[0];
+  __syncthreads();
+  // The first bin whose running total passes x (kCells: none); bin b's total
+  // is before[b + 1] - before[b], so the last usable bin is kCells - 1.
+  auto bin_of = [&](double x, bool inclusive) {
+    uint32_t mine = 0xFFFFFFFFu;
+#pragma unroll
+    for (int e = 1; e >= 0; --e) {
+      const int b = 2 * t + e;
+      if (b >= kCells) continue;
+      const double thru = rh.before[b + 1];
+      if (inclusive ? thru >= x : thru > x) mine = (uint32_t)b;
+    }
+    return min(block_min_u(mine, sh), (uint32_t)kCells);
+  };
+  auto bin_at = [&](float l) { return cell - grid_cell(l, scale); };
+
+  if (count) {
+    const uint32_t c = bin_of((double)a.top_k, true);
+    if (c == (uint32_t)kCells || rh.before[c + 1] > (double)CCAP) return none;
+    gather(n, l_of, [&](float l) { return bin_at(l) <= (float)c; }, tk);
+    rank_top((int)tk.n_cand, a.top_k, tk);
+    return tail_topk((uint32_t)a.top_k, a.temperature, a.top_p, r, tk);
+  }
+
+  // The top_p cut's bin and the bins the walk can stop in: its target is r
+  // times the kept weight, which lies between the cut bin's two ends.
+  const bool cutting = a.top_p < 1.0f;
+  uint32_t c = (uint32_t)kCells;
+  double kept_lo = total, kept_hi = total;
+  if (cutting) {
+    c = bin_of((double)a.top_p * total, true);
+    if (c == (uint32_t)kCells) return none;
+    kept_lo = rh.before[c];
+    kept_hi = rh.before[c + 1];
+  }
+  const uint32_t w0 = bin_of(r * kept_lo, false);
+  uint32_t w1 = bin_of(r * kept_hi, false);
+  if (cutting) w1 = min(w1, c);
+  if (w0 > w1 || w1 == (uint32_t)kCells || w1 - w0 > 5) return none;
+  // Their members in order; slot 7 is the cut bin, slot b - w0 the others.
+  gather(n, l_of, [&](float l) {
+    const float d = bin_at(l);
+    return (d >= (float)w0 && d <= (float)w1) || d == (float)c;
+  }, tk);
+  const int nc = (int)tk.n_cand;
+  if (nc > CCAP) return none;
+  rank_all(nc, tk);
+  if (t < 8) rh.first[t] = 0xFFFFFFFFu;
+  __syncthreads();
+  // Entries 2 t and 2 t + 1: value, bin, weight, and the weight before them.
+  double we[2];
+  uint32_t be[2];
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const int k = 2 * t + e;
+    we[e] = 0.0;
+    be[e] = 0u;
+    if (k < nc) {
+      const float l = key_value((uint32_t)(tk.sorted[k] >> 32));
+      be[e] = (uint32_t)bin_at(l);
+      we[e] = exp(((double)l - mxd) / T);
+      atomicMin(&rh.first[be[e] == c ? 7u : be[e] - w0], (uint32_t)k);
+    }
+  }
+  const double pre = block_scan_excl<double>(we[0] + we[1], sh.wave_d);
+  if (2 * t < nc) rh.pre[2 * t] = pre;
+  if (2 * t + 1 < nc) rh.pre[2 * t + 1] = pre + we[0];
+  __syncthreads();
+  // The row's running total through entry k.
+  auto through = [&](int e) {
+    const int k = 2 * t + e;
+    const uint32_t f = rh.first[be[e] == c ? 7u : be[e] - w0];
+    return rh.before[be[e]] + ((rh.pre[k] - rh.pre[f]) + we[e]);
+  };
+  auto first_entry = [&](auto test) {
+    uint32_t mine = 0xFFFFFFFFu;
+#pragma unroll
+    for (int e = 1; e >= 0; --e) {
+      const int k = 2 * t + e;
+      if (k < nc && we[e] != 0.0 && test(e, through(e))) mine = (uint32_t)k;
+    }
+    return block_min_u(mine, sh);
+  };
+  auto index_of = [&](uint32_t k) {
+    return 0xFFFFFFFFu - (uint32_t)(tk.sorted[k] & 0xFFFFFFFFull);
+  };
+  uint32_t cut = 0xFFFFFFFFu;
+  if (cutting) {
+    const double want = (double)a.top_p * total;
+    cut = first_entry([&](int e, double thru) { return be[e] == c && thru >= want; });
+    if (cut == 0xFFFFFFFFu) return none;
+    if ((uint32_t)(2 * t) == (cut & ~1u)) rh.target = cut & 1u ? through(1) : through(0);
+    __syncthreads();
+    total = rh.target;
+  }
+  const double stop = r * total;
+  const uint32_t pick = first_entry([&](int e, double thru) {
+    return (uint32_t)(2 * t + e) <= cut && thru > stop;
+  });
+  // No entry passes (r * total rounded up to total): the last kept one.
+  if (pick == 0xFFFFFFFFu) return cutting ? index_of(cut) : none;
+  return index_of(pick);
+}
+
+// `parts` > 0: k_sample_hist has left the row's bins in its workspace.
+__global__ __launch_bounds__(NT) void k_sample_rows(SampleArgs a, int parts) {
   extern __shared__ uint32_t bitmap[];
   __shared__ SampleShared sh;
   __shared__ TopKShared tk;
+  __shared__ RowHist rh;
   const int m = blockIdx.x, n = a.n;
   const float* row = a.logits + (size_t)m * a.row_stride;
   double* w = a.wbuf + (size_t)m * n;
 
-  // This row's seen ids (positions [s_lo, s_hi) of ids, a row of id_len
-  // entries) and draw, their loads issued together.
-  const uint32_t* ids = nullptr;
-  long id_len = 0;
-  int s_lo = 0, s_hi = 0;
+  SeenIds seen;
+  if (!row_seen(a, m, seen)) {
+    if (threadIdx.x == 0) a.active[m] = 0;
+    return;
+  }
   double r = 0.0;
-  if (a.tok) {
-    const int dn = a.done[m], st = a.start[m], p = a.pos[m];
-    const uint32_t c = a.count[m];
-    if (dn) {
-      if (threadIdx.x == 0) a.active[m] = 0;
-      return;
-    }
-    ids = a.hist + (size_t)m * a.hist_stride;
-    id_len = a.hist_stride;
-    s_lo = st;
-    s_hi = p > st ? p : st;
-    if (a.uniform) r = a.uniform[(size_t)c * gridDim.x + m];
-  } else {
-    if (a.seen) {
-      ids = a.seen + (size_t)m * a.seen_stride;
-      id_len = a.seen_stride;
-      s_hi = a.seen_len ? (int)min(a.seen_len[m], (uint32_t)a.seen_stride) : 0;
-    }
-    if (a.uniform) r = a.uniform[m];
-  }
-
-  // Bitmap of this row's seen ids (only if the penalty changes anything).
-  // The ids are read from their whole row (its extent is known) while the
-  // range is still being loaded.
-  const uint32_t* bm = nullptr;
-  if (a.penalty != 1.0f && ids) {
-    const int words = (n + 31) / 32;
-    for (long s0 = 0; s0 < id_len; s0 += 4 * NT) {
-      uint32_t v[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const long q = s0 + u * NT + threadIdx.x;
-        v[u] = q < id_len ? ids[q] : 0u;
-      }
-      if (s0 == 0) {
-        for (int k = threadIdx.x; k < words; k += NT) bitmap[k] = 0;
-        __syncthreads();
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const long q = s0 + u * NT + threadIdx.x;
-        if (q >= s_lo && q < s_hi && v[u] < (uint32_t)n) atomicOr(&bitmap[v[u] >> 5], 1u << (v[u] & 31));
-      }
-    }
-    if (id_len <= 0) {
-      for (int k = threadIdx.x; k < words; k += NT) bitmap[k] = 0;
-    }
-    __syncthreads();
-    bm = bitmap;
-  }
+  if (a.uniform) r = a.uniform[a.tok ? (size_t)a.count[m] * gridDim.x + m : m];
+  const uint32_t* bm = seen_bitmap(a, seen, bitmap);
   auto key_of = [&](int i) { return order_key(pen_logit(row, i, bm, a.penalty)); };
-
-  uint32_t pick;
-  bool picked = false;
-  const bool topk = a.temperature > 0.0f && a.top_k > 0 && a.top_k < n && a.top_k <= KCAP;
   auto l_at = [&](int i) { return pen_logit(row, i, bm, a.penalty); };
-  const int S = gridDim.y;
-  int nc = 0;
-  if (topk) {
-    // With S > 1 (the host splits only rows with topk, a.cnt, and
-    // S * (top_k + 1) <= n) this block takes part blockIdx.y of the row.
-    const int per = (n + S - 1) / S;
-    const int lo = min(n, (int)blockIdx.y * per), hi = min(n, lo + per);
-    if (lo < hi)
-      nc = topk_candidates(hi - lo, [&](int i) { return l_at(lo + i); }, (uint32_t)lo,
-                           (uint32_t)a.top_k, S > 1, sh, tk);
-  }
-  if (S > 1) {
-    // Its top_k (at most) to the row's workspace, then the row's last part
-    // to arrive merges them.
-    const int part = blockIdx.y;
-    const int L = nc;
-    unsigned long long* cand = reinterpret_cast<unsigned long long*>(w);
-    int* status = reinterpret_cast<int*>(cand + (size_t)S * a.top_k);
-    for (int t = threadIdx.x; t < L; t += NT)
-      __hip_atomic_store(cand + (size_t)part * a.top_k + t, tk.top[t], __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
-    if (threadIdx.x == 0)
-      __hip_atomic_store(status + part, L, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      const int done = __hip_atomic_fetch_add(a.cnt + m, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      sh.bcast_u[1] = done == S - 1;
-      if (done == S - 1)  // zero for the next launch
-        __hip_atomic_store(a.cnt + m, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    __syncthreads();
-    if (!sh.bcast_u[1]) return;
-    // Every part's status in one batch of loads (at most 16 parts).
-    int Lp[16];
-#pragma unroll
-    for (int q = 0; q < 16; ++q)
-      Lp[q] = q < S ? __hip_atomic_load(status + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
-    int total = 0;
-    bool fail = false;
-#pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      fail = fail || Lp[q] < 0;
-      total += Lp[q] > 0 ? Lp[q] : 0;
-    }
-    if (!fail && total >= a.top_k && total <= CCAP) {
-      // Entry e of the merged list: part q (the one whose prefix covers e),
-      // position e - prefix; a thread's entries (at most two) load at once.
-      unsigned long long got[CCAP / NT];
-#pragma unroll
-      for (int u = 0; u < CCAP / NT; ++u) {
-        const int e = threadIdx.x + u * NT;
-        int q = -1, base = 0, run = 0;
-#pragma unroll
-        for (int k = 0; k < 16; ++k) {
-          const int len = Lp[k] > 0 ? Lp[k] : 0;
-          if (q < 0 && e < run + len) {
-            q = k;
-            base = run;
-          }
-          run += len;
-        }
-        got[u] = q >= 0 ? __hip_atomic_load(cand + (size_t)q * a.top_k + (e - base),
-                                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                        : 0ull;
-      }
-#pragma unroll
-      for (int u = 0; u < CCAP / NT; ++u) {
-        const int e = threadIdx.x + u * NT;
-        if (e < total) tk.comp[e] = got[u];
-      }
-      __syncthreads();
-      rank_top(total, a.top_k, tk);
-      pick = tail_topk((uint32_t)a.top_k, a.temperature, a.top_p, r, tk);
-      picked = true;
-    }
-    // Otherwise this block takes the whole row on the radix path below.
-  } else if (topk && nc >= 0) {
+
+  uint32_t pick = (uint32_t)n;
+  if (parts > 0) {
+    pick = pick_binned(a, m, parts, l_at, r, sh, tk, rh);
+    __syncthreads();  // the radix path reuses the row's workspace and LDS
+  } else if (a.temperature > 0.0f && a.top_k > 0 && a.top_k < n && a.top_k <= KCAP &&
+             topk_candidates(n, l_at, (uint32_t)a.top_k, sh, tk) >= 0) {
     pick = tail_topk((uint32_t)a.top_k, a.temperature, a.top_p, r, tk);
-    picked = true;
   }
+  const bool picked = pick < (uint32_t)n;
   if (picked) {
   } else if (a.temperature <= 0.0f) {
     // sampling.rs:30-32, 83-91: first index of the maximum.
@@ -801,17 +1009,17 @@ hipError_t launch_sample_rows(const SampleArgs& a, int rows, hipStream_t s) {
                 a.max_new <= 0))
     return hipErrorInvalidValue;
   const size_t lds = a.penalty != 1.0f && (a.seen || a.tok) ? (size_t)(a.n + 31) / 32 * 4 : 0;
-  // Rows sampled with 0 < top_k <= 256 over parts of the vocabulary: about
-  // 256 blocks in all, at most 16 parts, each part's top_k and status within
-  // the row's workspace of n doubles, and all parts' top_k within CCAP.
-  int parts = 1;
-  if (a.cnt && rows <= kSampleCounters && a.temperature > 0.0f && a.top_k > 0 &&
-      a.top_k <= 256 && a.top_k < a.n) {
-    parts = std::min(AKH_SAMPLE_BLOCKS / 16, std::max(1, AKH_SAMPLE_BLOCKS / rows));
-    // The last block merges parts * top_k entries in its CCAP-entry buffer.
-    while (parts > 1 && ((long)parts * (a.top_k + 1) > a.n || (long)parts * a.top_k > CCAP)) --parts;
+  // Sampled rows long enough for at least one part's bins in their workspace of
+  // n doubles (top_k above KCAP stays on the radix path): about 256 blocks of
+  // bins in all, at most 16 parts a row (us for 32 x 50257 on MI355X, one block
+  // per row / binned: top_p alone 154 / 35.6, top_k 40 with top_p 36.5 / 32.6).
+  int parts = 0;
+  if (a.temperature > 0.0f && a.n >= kHistMin && (a.top_k <= KCAP || a.top_k >= a.n)) {
+    parts = std::min(kPartsMax, std::max(1, AKH_SAMPLE_BLOCKS / rows));
+    while (parts > 1 && ((long)parts * kHistMin > a.n || a.n / parts < NT)) --parts;
+    hipLaunchKernelGGL(k_sample_hist, dim3(rows, parts), dim3(NT), lds, s, a);
   }
-  hipLaunchKernelGGL(k_sample_rows, dim3(rows, parts), dim3(NT), lds, s, a);
+  hipLaunchKernelGGL(k_sample_rows, dim3(rows), dim3(NT), lds, s, a, parts);
   return hipGetLastError();
 }
 

@@ -156,3 +156,30 @@ def test_device_sampler_split_rows_edge_cases(backend, pkg, ora, rows, k):
     got = _device_sample(pkg, backend, l, 0.8, k, 0.95, 1.15, seen_rows, u)
     want = [ora.sample_token(l[i], 0.8, k, 0.95, seen_rows[i], 1.15, u[i]) for i in range(rows)]
     assert list(got) == want
+
+
+# Rows around the shortest that is binned (2050 ids: one part), over several
+# parts with a ragged last one, and more rows than parts; in each: no top_k, top_k
+# above and below what a bin holds, a row of equal logits (every id in one bin:
+# the radix path), one finite logit, steps of ties, a far lower half, draws at
+# both ends of [0, 1) and a grid far finer and far coarser than the logits.
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,n", [(7, 2049), (7, 2050), (7, 4101), (9, 20003), (300, 2500)])
+@pytest.mark.parametrize("t,k,p", [(0.8, 0, 0.95), (1.0, 0, 1.0), (0.01, 0, 0.5), (50.0, 0, 0.3),
+                                   (0.7, 1, 0.9), (1.2, 1000, 0.99), (0.9, 2000, 0.8)])
+def test_device_sampler_binned_rows(backend, pkg, ora, rows, n, t, k, p):
+    rng = np.random.default_rng(rows * n)
+    l = (rng.standard_normal((rows, n)) * 2.5).astype(np.float32)
+    l[0] = 1.25
+    l[1] = -np.inf
+    l[1, n - 1] = -3.0
+    l[2] = np.round(l[2] * 4) / 4
+    l[3, n // 2:] -= 200.0
+    l[4] += 1e6
+    u = rng.random(rows)
+    u[3], u[4], u[5], u[6] = 0.0, 0.5, 1.0 - 2.0 ** -53, 0.0
+    seen_rows = [rng.integers(0, n, int(rng.integers(0, 64))).astype(np.uint32) for _ in range(rows)]
+    got = _device_sample(pkg, backend, l, t, k, p, 1.15, seen_rows, u)
+    check = range(rows) if rows < 10 else list(range(8)) + [rows - 1]
+    want = [ora.sample_token(l[i], t, k, p, seen_rows[i], 1.15, u[i]) for i in check]
+    assert [int(got[i]) for i in check] == want
