@@ -1254,6 +1254,12 @@ __global__ __launch_bounds__(64 * AW) void k_dec_attn(DecAttnParams p) {
 #ifndef AKH_NORM_WIDE
 #define AKH_NORM_WIDE 1
 #endif
+#ifndef AKH_FEW_BLOCKS
+#define AKH_FEW_BLOCKS 256
+#endif
+#ifndef AKH_FEW_KMIN
+#define AKH_FEW_KMIN 96
+#endif
 template <int QPT, int NTH>
 __global__ __launch_bounds__(NTH) void k_rows_norm(RowsNormParams p) {
   static_assert(NTH == 256 || NTH == 512, "256 or 512 threads per row");
@@ -1329,6 +1335,193 @@ __global__ __launch_bounds__(NTH) void k_rows_norm(RowsNormParams p) {
           __fmul_rn(__fmul_rn(v.z, rs), g[i].z), __fmul_rn(__fmul_rn(v.w, rs), g[i].w));
     }
   }
+}
+
+// Y = A . W for M <= 4 rows on the VALU, W in 32-column float tiles: block
+// (tile, split) takes one tile's column sums over its range of K, thread (j,
+// g) column j and every eighth k-quad.  The step of one or two sequences is a
+// chain of memory round trips, so each block computes its own rows instead of
+// reading another kernel's: the RMSNorm of the residual plus the previous
+// GEMV's partial sums (block 0 stores the new residual), the merged attention
+// splits, or SiLU of ffn_up's sums.  Those loads go out first, then the
+// weights' (loads return in order: the rows are ready while the weights are
+// on their way).  Bound by launches and two memory round trips each: us on
+// MI355X, hall-1.0 at one sequence, before (with 2.3 per norm kernel) / here:
+// norm + qkv 6.0 / 4.2, out 4.0 / 3.3, norm + up 7.4 / 4.8, down 4.0 / 4.3; step
+// 378 / 298 at one sequence, 411 / 334 at two, 415 / 400 at four, where the rows'
+// partial sums take over (about 1 us per row and norm).
+template <int PRO, int M, int NI>  // NI: k-quads in flight per thread and pass
+__global__ __launch_bounds__(256) void k_dec_few(DecFewParams p) {
+  extern __shared__ float4 xs[];  // [M][quads]: whole rows (FEW_NORM) or the range's
+  __shared__ float red[4][M][32];
+  __shared__ float redw[M][4];
+  const int tid = threadIdx.x, j = tid & 31, g = tid >> 5, lane = tid & 63, wave = tid >> 6;
+  const int nq = p.K / 4;
+  const int per = (nq + p.splits - 1) / p.splits;
+  const int q0 = min(nq, (int)blockIdx.y * per), q1 = min(nq, q0 + per);
+  const float4* wt = reinterpret_cast<const float4*>(p.w) + (size_t)blockIdx.x * (p.Kp / 4) * 32 + j;
+  float4 w[NI];
+  auto load = [&](int q) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int k = q + g + 8 * i;
+      if (k < q1) {
+        const f32x4v v =
+            __builtin_nontemporal_load(reinterpret_cast<const f32x4v*>(wt + (size_t)k * 32));
+        w[i] = make_float4(v.x, v.y, v.z, v.w);
+      }
+    }
+  };
+  const bool gemv = p.w != nullptr;
+  auto load_first = [&]() {
+    asm volatile("" ::: "memory");
+    if (gemv && q0 < q1) load(q0);
+    asm volatile("" ::: "memory");
+  };
+  int qb = q0, stride = q1 - q0;  // xs holds quads from qb on, `stride` per row
+  if constexpr (PRO == FEW_NORM) {
+    qb = 0;
+    stride = nq;
+    // Thread t's quad of every row and its partial sums (kFewParts loads, those
+    // past nparts of the last again and not added), then the weights.
+    const int q = min(tid, nq - 1);
+    const bool live = tid < nq;
+    const float4 gn = reinterpret_cast<const float4*>(p.gain)[q];
+    float4 x[M], t[M][kFewParts];
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      const float* row = p.x + (size_t)m * p.K;
+      bool known = true;
+      if (p.ids) {
+        const uint32_t id = p.ids[m];
+        known = id < p.vocab;
+        row = p.table + (size_t)(known ? id : 0u) * p.K;
+      }
+      x[m] = reinterpret_cast<const float4*>(row)[q];
+      if (!known) x[m] = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (p.nparts > 0)
+#pragma unroll
+        for (int i = 0; i < kFewParts; ++i)
+          t[m][i] = *reinterpret_cast<const float4*>(
+              p.parts + (size_t)min(i, p.nparts - 1) * p.ps + (size_t)m * p.K + 4 * q);
+    }
+    load_first();
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (p.nparts > 0)
+#pragma unroll
+        for (int i = 0; i < kFewParts; ++i)
+          if (i < p.nparts) add4(sum, t[m][i]);
+      add4(x[m], sum);
+      const float4 v = x[m];
+      const float ss = wave_sum(live ? v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w : 0.f);
+      if (lane == 0) redw[m][wave] = ss;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      const float s = ((redw[m][0] + redw[m][1]) + redw[m][2]) + redw[m][3];
+      const float rs = 1.0f / sqrtf(s / (float)p.K + p.eps);
+      if (!live) continue;
+      const float4 v = x[m];
+      const float4 y = make_float4(
+          __fmul_rn(__fmul_rn(v.x, rs), gn.x), __fmul_rn(__fmul_rn(v.y, rs), gn.y),
+          __fmul_rn(__fmul_rn(v.z, rs), gn.z), __fmul_rn(__fmul_rn(v.w, rs), gn.w));
+      xs[m * nq + q] = y;
+      if (blockIdx.x == 0 && blockIdx.y == 0) {
+        if (p.x_out) reinterpret_cast<float4*>(p.x_out + (size_t)m * p.K)[q] = v;
+        if (p.xnt) reinterpret_cast<float4*>(p.xnt)[(size_t)q * 32 + m] = y;
+      }
+    }
+    if (!gemv) return;
+  } else {
+    // One quad of one row per thread (and round).
+    const int total = M * (q1 - q0);
+    float2 ml[kMaxAttnSplits];
+    float4 o[PRO == FEW_MERGE ? kMaxAttnSplits : kFewParts];
+    auto fetch = [&](int e) {
+      const int m = e / (q1 - q0), q = q0 + e - m * (q1 - q0);
+      if constexpr (PRO == FEW_MERGE) {
+        const int H = p.K / p.hd, hh = 4 * q / p.hd;
+#pragma unroll
+        for (int sp = 0; sp < kMaxAttnSplits; ++sp) {
+          const int c = min(sp, p.attn_splits - 1);
+          ml[sp] = p.ml[((size_t)c * H + hh) * p.rows + m];
+          o[sp] =
+              reinterpret_cast<const float4*>(p.out_t + (size_t)c * p.rows * p.K)[(size_t)q * 32 + m];
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < kFewParts; ++i)
+          o[i] = *reinterpret_cast<const float4*>(
+              p.parts + (size_t)min(i, p.nparts - 1) * p.ps + (size_t)m * p.K + 4 * q);
+      }
+    };
+    auto finish = [&](int e) {
+      float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+      if constexpr (PRO == FEW_MERGE) {
+        // Split states: maxima (log2 units) and sums per head, unnormalised o.
+        float mx = -INFINITY, L = 0.f;
+#pragma unroll
+        for (int sp = 0; sp < kMaxAttnSplits; ++sp) mx = fmaxf(mx, ml[sp].x);
+#pragma unroll
+        for (int sp = 0; sp < kMaxAttnSplits; ++sp) {
+          const float f =
+              sp >= p.attn_splits || ml[sp].x == -INFINITY ? 0.f : attn_exp(ml[sp].x - mx);
+          L += f * ml[sp].y;
+          v.x += f * o[sp].x;
+          v.y += f * o[sp].y;
+          v.z += f * o[sp].z;
+          v.w += f * o[sp].w;
+        }
+        const float inv = 1.0f / L;
+        v = make_float4(v.x * inv, v.y * inv, v.z * inv, v.w * inv);
+      } else {
+#pragma unroll
+        for (int i = 0; i < kFewParts; ++i)
+          if (i < p.nparts) add4(v, o[i]);
+        v = make_float4(silu_fast(v.x), silu_fast(v.y), silu_fast(v.z), silu_fast(v.w));
+      }
+      xs[e] = v;
+    };
+    if (total > 0) fetch(min(tid, total - 1));
+    load_first();
+    if (tid < total) finish(tid);
+    for (int e = tid + 256; e < total; e += 256) {
+      fetch(e);
+      finish(e);
+    }
+  }
+  __syncthreads();
+
+  float acc[M];
+#pragma unroll
+  for (int m = 0; m < M; ++m) acc[m] = 0.f;
+  for (int q = q0; q < q1; q += 8 * NI) {
+    if (q != q0) load(q);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int k = q + g + 8 * i;
+      if (k >= q1) break;
+#pragma unroll
+      for (int m = 0; m < M; ++m) {
+        const float4 a = xs[m * stride + k - qb];
+        acc[m] += w[i].x * a.x + w[i].y * a.y + w[i].z * a.z + w[i].w * a.w;
+      }
+    }
+  }
+  // The half-waves' sums, then the four waves' in order.
+#pragma unroll
+  for (int m = 0; m < M; ++m) {
+    const float v = xor_sum<32>(acc[m]);
+    if (lane < 32) red[wave][m][lane] = v;
+  }
+  __syncthreads();
+  const int m = tid >> 5, n = blockIdx.x * 32 + j;
+  if (m < M && n < p.N)
+    p.y[(size_t)blockIdx.y * p.ys + (size_t)m * p.N + n] =
+        ((red[0][m][j] + red[1][m][j]) + red[2][m][j]) + red[3][m][j];
 }
 
 __global__ __launch_bounds__(256) void k_argmax_final(
@@ -1928,6 +2121,45 @@ hipError_t launch_fill_kv_synthetic(void* kv, bool kv16, size_t planes, int len,
   const size_t blocks = std::min<size_t>((n + 255) / 256, 65536);
   hipLaunchKernelGGL(k_fill_kv_synthetic, dim3((unsigned)blocks), dim3(256), 0, s, kv, kv16,
                      planes, len, d, max_ctx, seed);
+  return hipGetLastError();
+}
+
+// At most one block per CU (hall-1.0 at one sequence, step us with 256 / 288
+// blocks: 301 / 320), at least 96 k each (64: no faster, more sums to read).
+int dec_few_splits(int K, int N) {
+  const int tiles = (N + 31) / 32;
+  return std::max(1, std::min({AKH_FEW_BLOCKS / tiles, K / AKH_FEW_KMIN, kFewParts}));
+}
+
+hipError_t launch_dec_few(const DecFewParams& p, int pro, hipStream_t s) {
+  if (p.M < 1 || p.M > kDecFewRows || p.K % 4 != 0 || p.K <= 0 || (p.w && p.splits < 1) ||
+      (pro == FEW_NORM && p.K > kDecFewMaxK) || (pro != FEW_NORM && !p.w))
+    return hipErrorInvalidValue;
+  const int nq = p.K / 4, per = p.w ? (nq + p.splits - 1) / p.splits : 0;
+  const dim3 g(p.w ? (p.N + 31) / 32 : 1, p.w ? p.splits : 1);
+  const size_t lds = (size_t)p.M * (pro == FEW_NORM ? nq : per) * sizeof(float4);
+#define AKH_FEW_NI(PRO, M)                                               \
+  if (per <= 32)                                                         \
+    hipLaunchKernelGGL((k_dec_few<PRO, M, 4>), g, dim3(256), lds, s, p);  \
+  else if (per <= 64)                                                    \
+    hipLaunchKernelGGL((k_dec_few<PRO, M, 8>), g, dim3(256), lds, s, p);  \
+  else                                                                   \
+    hipLaunchKernelGGL((k_dec_few<PRO, M, 12>), g, dim3(256), lds, s, p);
+#define AKH_FEW_GO(PRO)                                    \
+  switch (p.M) {                                           \
+    case 1: AKH_FEW_NI(PRO, 1) break;                      \
+    case 2: AKH_FEW_NI(PRO, 2) break;                      \
+    case 3: AKH_FEW_NI(PRO, 3) break;                      \
+    default: AKH_FEW_NI(PRO, 4) break;                     \
+  }
+  switch (pro) {
+    case FEW_NORM: AKH_FEW_GO(FEW_NORM) break;
+    case FEW_MERGE: AKH_FEW_GO(FEW_MERGE) break;
+    case FEW_SILU: AKH_FEW_GO(FEW_SILU) break;
+    default: return hipErrorInvalidValue;
+  }
+#undef AKH_FEW_GO
+#undef AKH_FEW_NI
   return hipGetLastError();
 }
 

@@ -399,6 +399,45 @@ hipError_t launch_fill_kv_synthetic(void* kv, bool kv16, size_t planes, int len,
 hipError_t launch_dec_attn(const DecAttnParams& p, int batch, int hd,
                            hipStream_t s, hipEvent_t t0 = nullptr, hipEvent_t t1 = nullptr);
 
+// Decode GEMVs of one to four sequences on float tiles (k_dec_few): five
+// kernels per layer, every block computing the rows it multiplies itself.
+// Activations are plain rows [M][.], partial sums [splits][M][N] (ps floats
+// per split).
+enum FewPro : int {
+  FEW_NORM = 0,   // RMSNorm of x + sum of parts (or of the embedding rows)
+  FEW_MERGE = 1,  // the merged attention splits
+  FEW_SILU = 2,   // SiLU of the sum of parts
+};
+struct DecFewParams {
+  const float* w;  // packed float tiles of Kp rows (none: FEW_NORM to xnt alone)
+  int M, K, N, Kp;
+  float* y;        // partial sums: split z, row m at y + z * ys + m * N
+  long ys;
+  int splits;      // dec_few_splits(K, N)
+  const float* parts;
+  int nparts;
+  long ps;
+  // FEW_NORM: x rows [M][K], or embedding rows of ids; the new residual goes
+  // to x_out, and without weights the normed rows to xnt (k-quad).
+  const float* x;
+  const uint32_t* ids;
+  const float* table;
+  uint32_t vocab;
+  const float* gain;
+  float eps;
+  float* x_out;
+  float* xnt;
+  // FEW_MERGE: the attention's splits (DecAttnParams::out_t, ml).
+  const float* out_t;
+  const float2* ml;
+  int attn_splits, hd, rows;
+};
+constexpr int kDecFewRows = 4;     // most sequences
+constexpr int kDecFewMaxK = 1024;  // widest row a block norms
+constexpr int kFewParts = 12;      // most splits, whose sums load at once
+int dec_few_splits(int K, int N);
+hipError_t launch_dec_few(const DecFewParams& p, int pro, hipStream_t s);
+
 // Per-row residual update + RMSNorm: x = table[ids[m]] (zero row if the id
 // is out of vocab), or src row (row0 + m * row_stride), or xt + the sum of
 // nparts row-major partial tiles [nparts][32][d]; xt <- x (k-quad) and

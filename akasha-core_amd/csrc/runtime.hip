@@ -1130,6 +1130,10 @@ struct akh_session {
   // two kernel boundaries it removes.  rcount holds the per-column-tile
   // block counters of the epilogues (zero between launches).
   bool fuse_out = false, fuse_down = false;
+  // One to four sequences (k_dec_few; null otherwise): the residual rows before
+  // and after a norm's sum, and each GEMV's partial sums.
+  float *few_x = nullptr, *few_qkv = nullptr, *few_out = nullptr, *few_up = nullptr,
+        *few_down = nullptr;
   float* ssq = nullptr;
   int* rcount = nullptr;
   float* logits = nullptr;  // [32, vocab]
@@ -1333,14 +1337,16 @@ hipError_t enqueue_qkv(akh_session* s, uint32_t l) {
   return launch_dec_gemm(p, DEC_CFG_QKV, s->be->stream);
 }
 
+bool few_rows(const akh_session* s);
+
 // q/k/v split + RoPE + cache append + cached attention
 // (inference_graphs.rs:385-456): one kernel.
 hipError_t enqueue_attn(akh_session* s, uint32_t l, hipEvent_t t0 = nullptr,
                         hipEvent_t t1 = nullptr) {
   const akh_model_config& c = s->m->cfg;
   DecAttnParams p{};
-  p.qkv = s->p_qkv;
-  p.nparts = s->ks_qkv;
+  p.qkv = few_rows(s) ? s->few_qkv : s->p_qkv;
+  p.nparts = few_rows(s) ? dec_few_splits((int)c.dim, 3 * (int)c.dim) : s->ks_qkv;
   p.rope = s->rope;
   p.kc = s->kv_at(l, 0);
   p.vc = s->kv_at(l, 1);
@@ -1445,6 +1451,126 @@ hipError_t enqueue_lm_head(akh_session* s) {
   return launch_dec_lm(p, s->be->num_cus, s->be->stream);
 }
 
+// Whether the step runs on the few-sequence GEMVs (k_dec_few): every
+// layer matrix in float tiles and no fused norm.
+bool few_rows(const akh_session* s) {
+  if (!s->few_x || s->fuse_out || s->fuse_down) return false;
+  for (uint32_t l = 0; l < s->m->cfg.num_layers; ++l)
+    for (int which : {W_QKV, W_OUT, W_UP, W_DOWN})
+      if (s->m->packed_layer(l, which).bf16) return false;
+  return true;
+}
+
+DecFewParams few_base(const akh_session* s, int K, int N) {
+  DecFewParams p{};
+  p.M = (int)s->B;
+  p.K = K;
+  p.N = N;
+  p.splits = dec_few_splits(K, N);
+  p.ys = (long)s->B * N;
+  p.eps = s->m->cfg.norm_eps;
+  return p;
+}
+
+void few_weights(DecFewParams& p, const PackedMatrix& pm) {
+  p.w = pm.w;
+  p.Kp = pm.rows;
+}
+
+// norm_1 + qkv_proj of layer l; the residual is the embedding (layer 0) or
+// row 0 of few_x plus the previous ffn_down's partial sums, and goes to row 1.
+hipError_t enqueue_few_qkv(akh_session* s, uint32_t l) {
+  const akh_model_config& c = s->m->cfg;
+  const int d = (int)c.dim;
+  DecFewParams p = few_base(s, d, 3 * d);
+  few_weights(p, s->m->packed_layer(l, W_QKV));
+  p.y = s->few_qkv;
+  p.ys = (long)s->rows() * 3 * d;  // the attention's partial tiles
+  p.gain = s->m->layer(l, W_NORM1);
+  if (l == 0) {
+    p.ids = s->tok;
+    p.table = s->m->embedding();
+    p.vocab = c.vocab_size;
+  } else {
+    p.x = s->few_x;
+    p.parts = s->few_down;
+    p.nparts = dec_few_splits((int)c.ffn_hidden, d);
+    p.ps = (long)s->B * d;
+  }
+  p.x_out = s->few_x + s->B * d;
+  return launch_dec_few(p, FEW_NORM, s->be->stream);
+}
+
+hipError_t enqueue_few_out(akh_session* s, uint32_t l) {
+  const akh_model_config& c = s->m->cfg;
+  const int d = (int)c.dim;
+  DecFewParams p = few_base(s, d, d);
+  few_weights(p, s->m->packed_layer(l, W_OUT));
+  p.y = s->few_out;
+  p.out_t = s->attn_t;
+  p.ml = s->attn_ml;
+  p.attn_splits = dec_attn_splits((int)s->B, (int)c.num_heads, (long)s->max_ctx, s->kv16);
+  p.hd = d / (int)c.num_heads;
+  p.rows = (int)s->rows();
+  return launch_dec_few(p, FEW_MERGE, s->be->stream);
+}
+
+// norm_2 + ffn_up; the residual (row 1 plus out_proj's sums) goes to row 0.
+hipError_t enqueue_few_up(akh_session* s, uint32_t l) {
+  const akh_model_config& c = s->m->cfg;
+  const int d = (int)c.dim;
+  DecFewParams p = few_base(s, d, (int)c.ffn_hidden);
+  few_weights(p, s->m->packed_layer(l, W_UP));
+  p.y = s->few_up;
+  p.gain = s->m->layer(l, W_NORM2);
+  p.x = s->few_x + s->B * d;
+  p.parts = s->few_out;
+  p.nparts = dec_few_splits(d, d);
+  p.ps = (long)s->B * d;
+  p.x_out = s->few_x;
+  return launch_dec_few(p, FEW_NORM, s->be->stream);
+}
+
+hipError_t enqueue_few_down(akh_session* s, uint32_t l) {
+  const akh_model_config& c = s->m->cfg;
+  const int d = (int)c.dim, F = (int)c.ffn_hidden;
+  DecFewParams p = few_base(s, F, d);
+  few_weights(p, s->m->packed_layer(l, W_DOWN));
+  p.y = s->few_down;
+  p.parts = s->few_up;
+  p.nparts = dec_few_splits(d, F);
+  p.ps = (long)s->B * F;
+  return launch_dec_few(p, FEW_SILU, s->be->stream);
+}
+
+// The final norm into the lm_head's rows.
+hipError_t enqueue_few_norm(akh_session* s) {
+  const akh_model_config& c = s->m->cfg;
+  const int d = (int)c.dim;
+  DecFewParams p = few_base(s, d, d);
+  p.gain = s->m->final_norm();
+  p.x = s->few_x;
+  p.parts = s->few_down;
+  p.nparts = dec_few_splits((int)c.ffn_hidden, d);
+  p.ps = (long)s->B * d;
+  p.xnt = s->xnt;
+  return launch_dec_few(p, FEW_NORM, s->be->stream);
+}
+
+hipError_t enqueue_few_body(akh_session* s) {
+  hipError_t e = hipSuccess;
+  for (uint32_t l = 0; l < s->m->cfg.num_layers && e == hipSuccess; ++l) {
+    e = enqueue_few_qkv(s, l);
+    if (e == hipSuccess) e = enqueue_attn(s, l);
+    if (e == hipSuccess) e = enqueue_few_out(s, l);
+    if (e == hipSuccess) e = enqueue_few_up(s, l);
+    if (e == hipSuccess) e = enqueue_few_down(s, l);
+  }
+  if (e == hipSuccess) e = enqueue_few_norm(s);
+  if (e == hipSuccess) e = enqueue_lm_head(s);
+  return e;
+}
+
 // One decode step of build_decode_layer (inference_graphs.rs:339-509) for
 // every sequence: embedding + norm_1, then per layer qkv GEMM, attention,
 // out GEMM, residual + norm_2, up GEMM, down GEMM, residual + next norm;
@@ -1454,6 +1580,7 @@ hipError_t enqueue_decode_generic(akh_session* s);
 
 hipError_t enqueue_decode_body(akh_session* s) {
   if (s->generic) return enqueue_decode_generic(s);
+  if (few_rows(s)) return enqueue_few_body(s);
   const akh_model_config& c = s->m->cfg;
   hipStream_t st = s->be->stream;
   RowsNormParams emb = norm_base(s, s->m->layer(0, W_NORM1));
@@ -1701,7 +1828,8 @@ extern "C" void akh_session_free(akh_session* s) {
                   s->logits, s->amax,   s->ssq,    s->rcount,
                   s->tok,    s->pos,    s->hist,   s->active, s->done,   s->gstart,
                   s->gcount, s->ggen,   s->guni,   s->gwbuf,  s->gx,     s->gxn,
-                  s->gqkv,   s->gattn,  s->gffn};
+                  s->gqkv,   s->gattn,  s->gffn,   s->few_x,  s->few_qkv, s->few_out,
+                  s->few_up, s->few_down};
   for (void* p : bufs)
     if (p) hipFree(p);
   delete s;
@@ -1782,6 +1910,16 @@ akh_status session_create(akh_model* m, uint32_t max_context_len, uint32_t batch
   alloc((void**)&s->p_up, (size_t)s->ks_up * R * F * 4);
   if (silu_own_kernel(s)) alloc((void**)&s->up_act, R * F * 4);
   alloc((void**)&s->p_down, (size_t)s->ks_down * R * d * 4);
+  if (batch <= (uint32_t)kDecFewRows && d <= (size_t)kDecFewMaxK) {
+    // k_dec_few's residual rows (two versions) and partial sums.
+    const size_t M = batch;
+    auto parts = [](size_t K, size_t N) { return (size_t)dec_few_splits((int)K, (int)N) * N; };
+    alloc((void**)&s->few_x, 2 * M * d * 4);
+    alloc((void**)&s->few_qkv, parts(d, 3 * d) * R * 4);
+    alloc((void**)&s->few_out, parts(d, d) * M * 4);
+    alloc((void**)&s->few_up, parts(d, F) * M * 4);
+    alloc((void**)&s->few_down, parts(F, d) * M * 4);
+  }
   if (dec_norm_fusable((int)d)) {  // for akh_session_set_fused_norm
     alloc((void**)&s->ssq, R * (d / 32) * 4);
     alloc((void**)&s->rcount, (d / 32) * sizeof(int));  // zeroed by alloc
@@ -2693,8 +2831,16 @@ extern "C" akh_status akh_session_time_decode_kernel(akh_session* s,
               "akh_session_time_decode_kernel: needs 1 <= cur_len < max_ctx");
   akh_backend* be = s->be;
   const uint32_t L = s->m->cfg.num_layers;
+  const bool few = few_rows(s);
   auto one = [&](uint32_t i) -> hipError_t {
     const uint32_t l = i % L;
+    if (few) switch (kernel) {
+        case 1: return enqueue_few_qkv(s, l);
+        case 2: return enqueue_few_out(s, l);
+        case 3: return enqueue_few_up(s, l);
+        case 4: return enqueue_few_down(s, l);
+        case 6: return enqueue_few_norm(s);
+      }
     switch (kernel) {
       case 0: return enqueue_attn(s, l);
       case 1: return enqueue_qkv(s, l);

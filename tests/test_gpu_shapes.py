@@ -13,6 +13,8 @@ cache (within 2e-2) and through generate's sampler.
 
 import dataclasses
 
+import dataclasses
+
 import numpy as np
 import pytest
 
@@ -158,3 +160,37 @@ def test_generic_shape_generate_and_errors(backend, pkg, ora):
         s.set_fused_norm(True)
     s.close()
     model.close()
+
+
+# One to four sequences decode on GEMVs that norm their own rows: the narrowest
+# row, one that leaves threads and the last K range partly idle, ffn widths of
+# one K range and of more k than a pass holds, the widest row, and the first
+# that is too wide (the batched kernels); ragged prompts, so positions differ.
+@pytest.mark.parametrize("batch,dim,heads,ffn", [
+    (1, 32, 2, 32), (2, 96, 3, 224), (3, 320, 5, 1280), (4, 768, 12, 3072), (1, 768, 6, 4128),
+    (2, 1024, 8, 96), (1, 1056, 11, 2080), (5, 96, 3, 224),
+])
+def test_few_sequences_decode_matches_oracle(backend, pkg, ora, batch, dim, heads, ffn):
+    cfg = dataclasses.replace(pkg.ModelConfig.new(173, dim, heads, 2, 40), ffn_hidden=ffn)
+    w = pkg.synthetic_weights(cfg, seed=91, std=0.05)
+    model = pkg.hip.Model(backend, cfg)
+    model.upload(w)
+    s = pkg.hip.Session(model, 40, batch)
+    few = batch <= 4 and dim <= 1024
+    assert s.decode_launches() == (5 * 2 + 3 if few else 7 * 2 + 3)
+    prompts = [pkg.synthetic_tokens(3 + 7 * b, 173, seed=92 + b) for b in range(batch)]
+    logits, nxt = s.prefill(prompts)
+    refs = [ora.OracleSession(cfg, w, 40) for _ in range(batch)]
+    want = [r.prefill(p) for r, p in zip(refs, prompts)]
+    for step in range(4):
+        for b in range(batch):
+            assert np.abs(logits[b] - want[b]).max() < 1e-3, (step, b)
+            assert int(nxt[b]) == ora.argmax(want[b]), (step, b)
+        want = [r.decode_step(int(t)) for r, t in zip(refs, nxt)]
+        logits, nxt = s.decode_step(None)
+    # The same steps replayed several to a graph.
+    s.truncate(3)
+    greedy = s.decode_greedy(9)
+    s.truncate(3)
+    assert np.array_equal(greedy, np.stack([s.decode_step(None)[1] for _ in range(9)]))
+    s.close()
