@@ -118,6 +118,20 @@ __device__ __forceinline__ uint32_t block_min_u(uint32_t v, SampleShared& sh) {
   return t;
 }
 
+// The value of the block's first thread that has one (0xFFFFFFFF: none).
+__device__ __forceinline__ uint32_t block_first_u(uint32_t v, SampleShared& sh) {
+  const unsigned long long has = __ballot(v != 0xFFFFFFFFu);
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int lead = has ? __ffsll((long long)has) - 1 : 0;
+  __syncthreads();
+  if (lane == lead) sh.wave_u[w] = v;
+  __syncthreads();
+  uint32_t t = 0xFFFFFFFFu;
+#pragma unroll
+  for (int k = NW - 1; k >= 0; --k) t = sh.wave_u[k] != 0xFFFFFFFFu ? sh.wave_u[k] : t;
+  return t;
+}
+
 __device__ __forceinline__ float block_max_f(float v, SampleShared& sh) {
   for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
   const int w = threadIdx.x >> 6;
@@ -305,9 +319,60 @@ __device__ __forceinline__ void rank_all(int nc, TopKShared& tk) {
 // divided out, and the walk r -= p.  The divisions, independent per element,
 // run in parallel; the folds and the walk, whose order fixes the bits, on one
 // thread.
+//
+// Up to 64 entries stay in the first wave: lane t holds entry t and the folds
+// read the lanes in order (the same operations in the same order, without an
+// LDS round trip per step).
+__device__ __forceinline__ uint32_t tail_topk_wave(int K, float temperature, float top_p, double r,
+                                                   TopKShared& tk) {
+  if (threadIdx.x < 64) {
+    const int lane = threadIdx.x;
+    const unsigned long long mine = tk.top[min(lane, K - 1)];
+    auto at = [](double v, int t) {
+      const unsigned long long u = __double_as_longlong(v);
+      return __longlong_as_double(
+          ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(u >> 32), t) << 32) |
+          (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, t));
+    };
+    const double mxd = (double)key_value((uint32_t)(tk.top[0] >> 32));
+    double p = exp(((double)key_value((uint32_t)(mine >> 32)) - mxd) / (double)temperature);
+    double sum = 0.0;
+    for (int t = 0; t < K; ++t) sum += at(p, t);
+    p /= sum;
+    int len = K;
+    if (top_p < 1.0f) {
+      double cum = 0.0;
+      for (int t = 0; t < K; ++t) {
+        cum += at(p, t);
+        if (cum >= (double)top_p) {
+          len = t + 1;
+          break;
+        }
+      }
+      double s2 = 0.0;
+      for (int t = 0; t < len; ++t) s2 += at(p, t);
+      p /= s2;
+    }
+    int k = len - 1;
+    double rr = r;
+    for (int t = 0; t < len; ++t) {
+      const double pt = at(p, t);
+      if (rr < pt) {
+        k = t;
+        break;
+      }
+      rr -= pt;
+    }
+    if (lane == 0) tk.pick = 0xFFFFFFFFu - (uint32_t)(tk.top[k] & 0xFFFFFFFFull);
+  }
+  __syncthreads();
+  return tk.pick;
+}
+
 __device__ __forceinline__ uint32_t tail_topk(uint32_t top_k, float temperature, float top_p,
                                               double r, TopKShared& tk) {
   const int K = (int)top_k;
+  if (K <= 64) return tail_topk_wave(K, temperature, top_p, r, tk);
   const double mxd = (double)key_value((uint32_t)(tk.top[0] >> 32));
   for (int t = threadIdx.x; t < K; t += NT)
     tk.prob[t] = exp(((double)key_value((uint32_t)(tk.top[t] >> 32)) - mxd) / (double)temperature);
@@ -578,7 +643,9 @@ __device__ __forceinline__ bool row_seen(const SampleArgs& a, int m, SeenIds& s)
 // (and of the row) are the kCells cells from its maximum's down, bin d the
 // cell d below.  What lies further below is only in the part's total.  The
 // row's workspace holds kBins doubles per part (f64 weights relative to the
-// part's maximum, or uint32 counts), then a header per part.
+// part's maximum, or uint32 counts), then a header per part, then with a
+// penalty the penalised logits, which the row's block reads instead of looking
+// every id up again.
 // ---------------------------------------------------------------------------
 constexpr int kCells = kBins - 1;
 constexpr int kPartsMax = 16;
@@ -589,7 +656,11 @@ struct PartHead {
 };
 static_assert(sizeof(PartHead) == 2 * sizeof(double), "two doubles of the row's workspace");
 static_assert(kBins == 2 * NT && CCAP == 2 * NT, "two bins and two list entries per thread");
-constexpr int kHistMin = kBins + 2;  // ids: one part's bins and header
+// Doubles of the workspace before the penalised logits.
+__host__ __device__ constexpr long hist_doubles(int parts) { return (long)parts * (kBins + 2); }
+// Shortest row: one part's bins, its header and the penalised logits (4 bytes
+// an id, of the workspace's 8).
+constexpr int kHistMin = 2 * (kBins + 2);
 
 // About 64 cells per logit or 48 per unit of l / T, whichever is finer: cells
 // of ~150 ids at the densest of 50257 logits N(0, 2^2), and 2047 cells reach
@@ -625,6 +696,16 @@ __global__ __launch_bounds__(NT) void k_sample_hist(SampleArgs a) {
     for (int u = 0; u < U; ++u) f(v[u]);
     for (int i = U * NT + (int)threadIdx.x; i < len; i += NT) f(l_at(i));
   };
+  double* base = a.wbuf + (size_t)m * a.n;
+  if (bm) {
+    float* copy = reinterpret_cast<float*>(base + hist_doubles(parts)) + lo;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i = u * NT + (int)threadIdx.x;
+      if (i < len) copy[i] = v[u];
+    }
+    for (int i = U * NT + (int)threadIdx.x; i < len; i += NT) copy[i] = l_at(i);
+  }
   float mxv = -INFINITY;
   uint32_t nan = 0;
   each([&](float l) {
@@ -657,7 +738,6 @@ __global__ __launch_bounds__(NT) void k_sample_hist(SampleArgs a) {
     });
   }
   const double total = block_sum_d(own, sh);  // its barriers complete the bins
-  double* base = a.wbuf + (size_t)m * a.n;
   if (!bad && !empty) {
     double* bins = base + (size_t)part * kBins;
     for (int b = threadIdx.x; b < kBins; b += NT) {
@@ -673,10 +753,9 @@ struct RowHist {
   double before[kBins];  // weight (or count) of the bins above
   float part_max[kPartsMax];
   double part_f[kPartsMax];
-  uint32_t first[8];     // list position of a bin's first entry
+  uint32_t first[2];     // list position of a run's first entry
   double pre[CCAP];      // weight of the list's entries before each
   double target;
-  uint32_t lo, hi, cut;
 };
 
 // The pick of row m from its parts' bins, or n where the radix path must
@@ -737,7 +816,7 @@ __device__ __forceinline__ uint32_t pick_binned(const SampleArgs& a, int m, int 
       const double thru = rh.before[b + 1];
       if (inclusive ? thru >= x : thru > x) mine = (uint32_t)b;
     }
-    return min(block_min_u(mine, sh), (uint32_t)kCells);
+    return min(block_first_u(mine, sh), (uint32_t)kCells);
   };
   auto bin_at = [&](float l) { return cell - grid_cell(l, scale); };
 
@@ -763,8 +842,9 @@ __device__ __forceinline__ uint32_t pick_binned(const SampleArgs& a, int m, int 
   const uint32_t w0 = bin_of(r * kept_lo, false);
   uint32_t w1 = bin_of(r * kept_hi, false);
   if (cutting) w1 = min(w1, c);
-  if (w0 > w1 || w1 == (uint32_t)kCells || w1 - w0 > 5) return none;
-  // Their members in order; slot 7 is the cut bin, slot b - w0 the others.
+  if (w0 > w1 || w1 == (uint32_t)kCells) return none;
+  // Their members in order: the walk's bins are one run of the order, the cut
+  // bin, where it lies below them, another.
   gather(n, l_of, [&](float l) {
     const float d = bin_at(l);
     return (d >= (float)w0 && d <= (float)w1) || d == (float)c;
@@ -772,7 +852,7 @@ __device__ __forceinline__ uint32_t pick_binned(const SampleArgs& a, int m, int 
   const int nc = (int)tk.n_cand;
   if (nc > CCAP) return none;
   rank_all(nc, tk);
-  if (t < 8) rh.first[t] = 0xFFFFFFFFu;
+  if (t < 2) rh.first[t] = 0xFFFFFFFFu;
   __syncthreads();
   // Entries 2 t and 2 t + 1: value, bin, weight, and the weight before them.
   double we[2];
@@ -786,7 +866,7 @@ __device__ __forceinline__ uint32_t pick_binned(const SampleArgs& a, int m, int 
       const float l = key_value((uint32_t)(tk.sorted[k] >> 32));
       be[e] = (uint32_t)bin_at(l);
       we[e] = exp(((double)l - mxd) / T);
-      atomicMin(&rh.first[be[e] == c ? 7u : be[e] - w0], (uint32_t)k);
+      atomicMin(&rh.first[be[e] > w1 ? 1 : 0], (uint32_t)k);
     }
   }
   const double pre = block_scan_excl<double>(we[0] + we[1], sh.wave_d);
@@ -796,8 +876,8 @@ __device__ __forceinline__ uint32_t pick_binned(const SampleArgs& a, int m, int 
   // The row's running total through entry k.
   auto through = [&](int e) {
     const int k = 2 * t + e;
-    const uint32_t f = rh.first[be[e] == c ? 7u : be[e] - w0];
-    return rh.before[be[e]] + ((rh.pre[k] - rh.pre[f]) + we[e]);
+    const bool low = be[e] > w1;
+    return rh.before[low ? c : w0] + ((rh.pre[k] - rh.pre[rh.first[low ? 1 : 0]]) + we[e]);
   };
   auto first_entry = [&](auto test) {
     uint32_t mine = 0xFFFFFFFFu;
@@ -806,7 +886,7 @@ __device__ __forceinline__ uint32_t pick_binned(const SampleArgs& a, int m, int 
       const int k = 2 * t + e;
       if (k < nc && we[e] != 0.0 && test(e, through(e))) mine = (uint32_t)k;
     }
-    return block_min_u(mine, sh);
+    return block_first_u(mine, sh);
   };
   auto index_of = [&](uint32_t k) {
     return 0xFFFFFFFFu - (uint32_t)(tk.sorted[k] & 0xFFFFFFFFull);
@@ -846,18 +926,20 @@ __global__ __launch_bounds__(NT) void k_sample_rows(SampleArgs a, int parts) {
   }
   double r = 0.0;
   if (a.uniform) r = a.uniform[a.tok ? (size_t)a.count[m] * gridDim.x + m : m];
-  const uint32_t* bm = seen_bitmap(a, seen, bitmap);
-  auto key_of = [&](int i) { return order_key(pen_logit(row, i, bm, a.penalty)); };
-  auto l_at = [&](int i) { return pen_logit(row, i, bm, a.penalty); };
-
   uint32_t pick = (uint32_t)n;
   if (parts > 0) {
-    pick = pick_binned(a, m, parts, l_at, r, sh, tk, rh);
-    __syncthreads();  // the radix path reuses the row's workspace and LDS
-  } else if (a.temperature > 0.0f && a.top_k > 0 && a.top_k < n && a.top_k <= KCAP &&
-             topk_candidates(n, l_at, (uint32_t)a.top_k, sh, tk) >= 0) {
-    pick = tail_topk((uint32_t)a.top_k, a.temperature, a.top_p, r, tk);
+    const float* src = a.penalty == 1.0f || !seen.ids
+                           ? row
+                           : reinterpret_cast<const float*>(w + hist_doubles(parts));
+    pick = pick_binned(a, m, parts, [&](int i) { return src[i]; }, r, sh, tk, rh);
+    __syncthreads();  // the other paths reuse the row's workspace and LDS
   }
+  const uint32_t* bm = pick < (uint32_t)n ? nullptr : seen_bitmap(a, seen, bitmap);
+  auto key_of = [&](int i) { return order_key(pen_logit(row, i, bm, a.penalty)); };
+  auto l_at = [&](int i) { return pen_logit(row, i, bm, a.penalty); };
+  if (parts <= 0 && a.temperature > 0.0f && a.top_k > 0 && a.top_k < n && a.top_k <= KCAP &&
+      topk_candidates(n, l_at, (uint32_t)a.top_k, sh, tk) >= 0)
+    pick = tail_topk((uint32_t)a.top_k, a.temperature, a.top_p, r, tk);
   const bool picked = pick < (uint32_t)n;
   if (picked) {
   } else if (a.temperature <= 0.0f) {
@@ -1012,11 +1094,11 @@ hipError_t launch_sample_rows(const SampleArgs& a, int rows, hipStream_t s) {
   // Sampled rows long enough for at least one part's bins in their workspace of
   // n doubles (top_k above KCAP stays on the radix path): about 256 blocks of
   // bins in all, at most 16 parts a row (us for 32 x 50257 on MI355X, one block
-  // per row / binned: top_p alone 154 / 35.6, top_k 40 with top_p 36.5 / 32.6).
+  // per row / binned: top_p alone 154 / 35.2, top_k 40 with top_p 36.5 / 30.5).
   int parts = 0;
   if (a.temperature > 0.0f && a.n >= kHistMin && (a.top_k <= KCAP || a.top_k >= a.n)) {
     parts = std::min(kPartsMax, std::max(1, AKH_SAMPLE_BLOCKS / rows));
-    while (parts > 1 && ((long)parts * kHistMin > a.n || a.n / parts < NT)) --parts;
+    while (parts > 1 && (2 * hist_doubles(parts) > a.n || a.n / parts < NT)) --parts;
     hipLaunchKernelGGL(k_sample_hist, dim3(rows, parts), dim3(NT), lds, s, a);
   }
   hipLaunchKernelGGL(k_sample_rows, dim3(rows), dim3(NT), lds, s, a, parts);
