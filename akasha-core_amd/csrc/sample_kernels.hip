@@ -51,6 +51,9 @@ namespace {
 #ifndef AKH_SAMPLE_BLOCKS
 #define AKH_SAMPLE_BLOCKS 256
 #endif
+#ifndef AKH_GATHER_U
+#define AKH_GATHER_U 25
+#endif
 constexpr int NT = AKH_SAMPLE_NT;  // threads per row (per part of a binned row)
 constexpr int NW = NT / 64;     // waves per block
 
@@ -133,7 +136,7 @@ __device__ __forceinline__ uint32_t block_first_u(uint32_t v, SampleShared& sh) 
 }
 
 __device__ __forceinline__ float block_max_f(float v, SampleShared& sh) {
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
+  v = wave_max(v);
   const int w = threadIdx.x >> 6;
   __syncthreads();
   if ((threadIdx.x & 63) == 0) sh.wave_f[w] = v;
@@ -465,6 +468,54 @@ __device__ void reduce_counts(const uint32_t (&c)[NTH], uint32_t base, TopKShare
   __syncthreads();
 }
 
+// The smallest float whose grid cell is at least `cell` (floor(l * scale),
+// which grows with l).
+__device__ __forceinline__ float cell_low(float cell, float scale) {
+  auto at_least = [&](float l) { return floorf(__fmul_rn(l, scale)) >= cell; };
+  auto step = [](float l, int by) {  // the by-th float above or below l
+    const uint32_t u = __float_as_uint(l);
+    const int o = (u & 0x80000000u) ? -(int)(u & 0x7FFFFFFFu) : (int)u;
+    const int v = o + by;
+    return __uint_as_float(v < 0 ? 0x80000000u | (uint32_t)-v : (uint32_t)v);
+  };
+  float l = cell / scale;
+  while (at_least(l)) l = step(l, -1);
+  while (!at_least(l)) l = step(l, 1);
+  return l;
+}
+
+// tk.comp[0 .. tk.n_cand) = the elements of src[0 .. n) in [a0, a1) or [b0, b1),
+// in any order (n_cand counts those past CCAP too).  A chunk's test leaves a
+// bit per id, and the few that are set are appended in a loop: a dispatch
+// starts with cold instruction caches, and straight-line code for every id of
+// a chunk cost more to fetch than to run (the row kernel on 32 x 50257: 25 us
+// so, 21 here; 25 ids a thread, two rounds of loads, against 16: 1 to 2 us).
+__device__ __forceinline__ void gather_ranges(const float* src, int n, float a0, float a1, float b0,
+                                              float b1, TopKShared& tk) {
+  constexpr int UN = AKH_GATHER_U;
+  if (threadIdx.x == 0) tk.n_cand = 0;
+  __syncthreads();
+  for (int c0 = 0; c0 < n; c0 += NT * UN) {
+    const int i0 = c0 + (int)threadIdx.x;
+    float v[UN];
+#pragma unroll
+    for (int u = 0; u < UN; ++u) v[u] = src[min(i0 + u * NT, n - 1)];
+    uint32_t hits = 0;
+#pragma unroll
+    for (int u = 0; u < UN; ++u)
+      if ((v[u] >= a0 && v[u] < a1) || (v[u] >= b0 && v[u] < b1)) hits |= 1u << u;
+    while (hits) {
+      const int i = i0 + (__ffs((int)hits) - 1) * NT;
+      hits &= hits - 1;
+      if (i >= n) break;
+      const uint32_t slot = atomicAdd(&tk.n_cand, 1u);
+      if (slot < (uint32_t)CCAP)
+        tk.comp[slot] = ((unsigned long long)order_key(src[i]) << 32) | (0xFFFFFFFFu - (uint32_t)i);
+    }
+  }
+  __syncthreads();
+}
+
 // tk.comp[0 .. tk.n_cand) = the elements of the row that `take` accepts, in
 // any order (n_cand counts those past CCAP too).
 template <typename LFn, typename TakeFn>
@@ -719,7 +770,7 @@ __global__ __launch_bounds__(NT) void k_sample_hist(SampleArgs a) {
   const float mx = block_max_f(mxv, sh);
   const float scale = grid_scale(a.temperature);
   const bool empty = mx == -INFINITY;
-  const bool bad = block_sum_u(nan, sh) != 0 || mx == INFINITY ||
+  const bool bad = __syncthreads_or((int)nan) || mx == INFINITY ||
                    (!empty && !(fabsf(mx) * scale < 0x1p30f));
   double own = 0.0;
   if (!bad && !empty) {
@@ -751,7 +802,7 @@ __global__ __launch_bounds__(NT) void k_sample_hist(SampleArgs a) {
 
 struct RowHist {
   double before[kBins];  // weight (or count) of the bins above
-  float part_max[kPartsMax];
+  PartHead head[kPartsMax];
   double part_f[kPartsMax];
   uint32_t first[2];     // list position of a run's first entry
   double pre[CCAP];      // weight of the list's entries before each
@@ -760,9 +811,8 @@ struct RowHist {
 
 // The pick of row m from its parts' bins, or n where the radix path must
 // decide.  Every thread of the block calls it.
-template <typename LFn>
-__device__ __forceinline__ uint32_t pick_binned(const SampleArgs& a, int m, int parts, LFn l_of,
-                                                double r, SampleShared& sh, TopKShared& tk,
+__device__ __forceinline__ uint32_t pick_binned(const SampleArgs& a, int m, int parts,
+                                                const float* src, double r, SampleShared& sh, TopKShared& tk,
                                                 RowHist& rh) {
   const uint32_t none = (uint32_t)a.n;
   const int n = a.n, t = threadIdx.x;
@@ -770,35 +820,50 @@ __device__ __forceinline__ uint32_t pick_binned(const SampleArgs& a, int m, int 
   const float scale = grid_scale(a.temperature);
   const double* base = a.wbuf + (size_t)m * n;
   const PartHead* head = reinterpret_cast<const PartHead*>(base + (size_t)parts * kBins);
+  if (t < parts) rh.head[t] = head[t];
+  __syncthreads();
   float mx = -INFINITY;
   int bad = 0;
   for (int q = 0; q < parts; ++q) {
-    mx = fmaxf(mx, head[q].max);
-    bad |= head[q].bad;
+    mx = fmaxf(mx, rh.head[q].max);
+    bad |= rh.head[q].bad;
   }
   if (bad || mx == -INFINITY) return none;  // uniform
   const double mxd = (double)mx, T = (double)a.temperature;
-  if (t < parts) {
-    rh.part_max[t] = head[t].max;
-    rh.part_f[t] = head[t].max == -INFINITY ? 0.0 : exp(((double)head[t].max - mxd) / T);
-  }
+  if (t < parts)
+    rh.part_f[t] = rh.head[t].max == -INFINITY ? 0.0 : exp(((double)rh.head[t].max - mxd) / T);
   __syncthreads();
   double total = 0.0;
-  for (int q = 0; q < parts; ++q) total += rh.part_f[q] * head[q].total;
+  for (int q = 0; q < parts; ++q) total += rh.part_f[q] * rh.head[q].total;
 
   // Thread t's bins 2 t and 2 t + 1 over the parts, then every bin's total
   // above it.
   const float cell = grid_cell(mx, scale);
+  // Eight parts' loads at a time, without branches between them (a part past
+  // the last, an empty one and bins outside a part read bin 0 and count 0).
   double v[2] = {0.0, 0.0};
-  for (int q = 0; q < parts; ++q) {
-    const float off = cell - grid_cell(rh.part_max[q], scale);  // inf: an empty part
-    if (!(off < (float)kCells)) continue;
+  for (int p0 = 0; p0 < parts; p0 += 8) {
+    double x[8][2];
+    bool in[8][2];
 #pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      const int b = 2 * t + e - (int)off;
-      if (b < 0 || 2 * t + e >= kCells) continue;
-      v[e] += count ? (double)reinterpret_cast<const uint32_t*>(base + (size_t)q * kBins)[b]
-                    : rh.part_f[q] * base[(size_t)q * kBins + b];
+    for (int u = 0; u < 8; ++u) {
+      const int q = min(p0 + u, parts - 1);
+      const float off = cell - grid_cell(rh.head[q].max, scale);  // inf: an empty part
+      const int b0 = off < (float)kCells ? 2 * t - (int)off : -kBins;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        in[u][e] = p0 + u < parts && b0 + e >= 0 && 2 * t + e < kCells;
+        const int b = in[u][e] ? b0 + e : 0;
+        x[u][e] = count ? (double)reinterpret_cast<const uint32_t*>(base + (size_t)q * kBins)[b]
+                        : base[(size_t)q * kBins + b];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const double f = count ? 1.0 : rh.part_f[min(p0 + u, parts - 1)];
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+        if (in[u][e]) v[e] += f * x[u][e];
     }
   }
   const double above = block_scan_excl<double>(v[0] + v[1], sh.wave_d);
@@ -823,7 +888,8 @@ __device__ __forceinline__ uint32_t pick_binned(const SampleArgs& a, int m, int 
   if (count) {
     const uint32_t c = bin_of((double)a.top_k, true);
     if (c == (uint32_t)kCells || rh.before[c + 1] > (double)CCAP) return none;
-    gather(n, l_of, [&](float l) { return bin_at(l) <= (float)c; }, tk);
+    const float lo = cell_low(cell - (float)c, scale);
+    gather_ranges(src, n, lo, INFINITY, INFINITY, INFINITY, tk);
     rank_top((int)tk.n_cand, a.top_k, tk);
     return tail_topk((uint32_t)a.top_k, a.temperature, a.top_p, r, tk);
   }
@@ -845,10 +911,11 @@ __device__ __forceinline__ uint32_t pick_binned(const SampleArgs& a, int m, int 
   if (w0 > w1 || w1 == (uint32_t)kCells) return none;
   // Their members in order: the walk's bins are one run of the order, the cut
   // bin, where it lies below them, another.
-  gather(n, l_of, [&](float l) {
-    const float d = bin_at(l);
-    return (d >= (float)w0 && d <= (float)w1) || d == (float)c;
-  }, tk);
+  auto low_of = [&](uint32_t b) { return cell_low(cell - (float)b, scale); };
+  const bool apart = cutting && c > w1;
+  const float w_hi = w0 == 0 ? INFINITY : low_of(w0 - 1);
+  gather_ranges(src, n, low_of(w1), w_hi, apart ? low_of(c) : INFINITY,
+                apart ? low_of(c - 1) : INFINITY, tk);
   const int nc = (int)tk.n_cand;
   if (nc > CCAP) return none;
   rank_all(nc, tk);
@@ -931,7 +998,7 @@ __global__ __launch_bounds__(NT) void k_sample_rows(SampleArgs a, int parts) {
     const float* src = a.penalty == 1.0f || !seen.ids
                            ? row
                            : reinterpret_cast<const float*>(w + hist_doubles(parts));
-    pick = pick_binned(a, m, parts, [&](int i) { return src[i]; }, r, sh, tk, rh);
+    pick = pick_binned(a, m, parts, src, r, sh, tk, rh);
     __syncthreads();  // the other paths reuse the row's workspace and LDS
   }
   const uint32_t* bm = pick < (uint32_t)n ? nullptr : seen_bitmap(a, seen, bitmap);
@@ -1094,7 +1161,7 @@ hipError_t launch_sample_rows(const SampleArgs& a, int rows, hipStream_t s) {
   // Sampled rows long enough for at least one part's bins in their workspace of
   // n doubles (top_k above KCAP stays on the radix path): about 256 blocks of
   // bins in all, at most 16 parts a row (us for 32 x 50257 on MI355X, one block
-  // per row / binned: top_p alone 154 / 35.2, top_k 40 with top_p 36.5 / 30.5).
+  // per row / binned: top_p alone 164 / 32.6, top_k 40 with top_p 36.8 / 28.8).
   int parts = 0;
   if (a.temperature > 0.0f && a.n >= kHistMin && (a.top_k <= KCAP || a.top_k >= a.n)) {
     parts = std::min(kPartsMax, std::max(1, AKH_SAMPLE_BLOCKS / rows));
