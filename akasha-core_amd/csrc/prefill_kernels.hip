@@ -1475,10 +1475,12 @@ __global__ __launch_bounds__(64 * WM * WN * KG, 2) void k_gemm_h3(GemmParams p) 
 // stores its partial sums to p.c + z M N (GEMM_STORE; the caller's next norm
 // adds them).  Waves add in order, so results are reproducible.  At 64 rows it
 // is bound by a few memory round trips in a row: 64 x 2304 x 768 26 us on 128
-// x 128 tiles, 7.9 here; 64 x 768 x 3072 88 and 6.5 (8 ranges).
+// x 128 tiles, 8.4 here; 64 x 768 x 3072 88 and 6.8 (8 ranges).  One row tile
+// takes four waves with six units in flight (eight waves with four: 10.3 and
+// 7.6), two take eight with two (four with four to eight: 5 to 15 % slower).
 template <int EPI, int TR, int W, int D>
 __global__ __launch_bounds__(64 * W, 2) void k_gemm_h3k(GemmParams p) {
-  static_assert(D % 2 == 0 && W >= 4 * TR, "whole pairs of units in flight; four rows per wave");
+  static_assert(D % 2 == 0, "whole pairs of units in flight");
   __shared__ __align__(16) float red[W][TR * 2][4][64][4];
 
   const int M = p.M, N = p.N, K = p.K;
@@ -1546,8 +1548,8 @@ __global__ __launch_bounds__(64 * W, 2) void k_gemm_h3k(GemmParams p) {
     }
   }
 
-  // Every wave's sums to LDS, then wave w adds four rows of tile pair w / 4
-  // over the waves and runs their epilogue.
+  // Every wave's sums to LDS, then wave w adds four rows of tile pair x / 4 over
+  // the waves and runs their epilogue, for x = w, w + W, ...
 #pragma unroll
   for (int a = 0; a < TR; ++a)
 #pragma unroll
@@ -1560,18 +1562,22 @@ __global__ __launch_bounds__(64 * W, 2) void k_gemm_h3k(GemmParams p) {
                         acc[a][t][4 * q + 2] + cor[a][t][4 * q + 2] * 0x1p-11f,
                         acc[a][t][4 * q + 3] + cor[a][t][4 * q + 3] * 0x1p-11f);
   __syncthreads();
-  if (w >= 4 * TR) return;
-  const int a = w >> 2, q = w & 3;
-  float v0[4] = {0.f, 0.f, 0.f, 0.f}, v1[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int i = 0; i < W; ++i) {
-    const float4 x = *reinterpret_cast<const float4*>(red[i][2 * a][q][lane]);
-    const float4 y = *reinterpret_cast<const float4*>(red[i][2 * a + 1][q][lane]);
-    v0[0] += x.x, v0[1] += x.y, v0[2] += x.z, v0[3] += x.w;
-    v1[0] += y.x, v1[1] += y.y, v1[2] += y.z, v1[3] += y.w;
-  }
   p.c += (size_t)z * M * N;
-  if (!epi_h3<EPI, 4>(p, M, N, m0 + 32 * a, g * 64 + 2 * j, v0, v1, 4 * q)) *p.range_flag = 1;
+  bool finite = true;
+#pragma unroll
+  for (int x = w; x < 4 * TR; x += W) {
+    const int a = x >> 2, q = x & 3;
+    float v0[4] = {0.f, 0.f, 0.f, 0.f}, v1[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < W; ++i) {
+      const float4 s = *reinterpret_cast<const float4*>(red[i][2 * a][q][lane]);
+      const float4 y = *reinterpret_cast<const float4*>(red[i][2 * a + 1][q][lane]);
+      v0[0] += s.x, v0[1] += s.y, v0[2] += s.z, v0[3] += s.w;
+      v1[0] += y.x, v1[1] += y.y, v1[2] += y.z, v1[3] += y.w;
+    }
+    finite = epi_h3<EPI, 4>(p, M, N, m0 + 32 * a, g * 64 + 2 * j, v0, v1, 4 * q) && finite;
+  }
+  if (!finite) *p.range_flag = 1;
 }
 
 // k_rows_rmsnorm with its rows into A's planes: a wave per row, eight rows per
@@ -3229,8 +3235,8 @@ hipError_t launch_gemm_h3(const GemmParams& p, int epi, hipStream_t s) {
 #define AKH_H3_GO(E)                                                                          \
   switch (plan.kind) {                                                                        \
     case H3_ROW1:                                                                             \
-      hipLaunchKernelGGL((k_gemm_h3k<E, 1, 8, 4>), dim3((p.M + 31) / 32, (p.N + 63) / 64, gz), \
-                         dim3(512), 0, s, q);                                                 \
+      hipLaunchKernelGGL((k_gemm_h3k<E, 1, 4, 6>), dim3((p.M + 31) / 32, (p.N + 63) / 64, gz), \
+                         dim3(256), 0, s, q);                                                 \
       break;                                                                                  \
     case H3_ROW2:                                                                             \
       hipLaunchKernelGGL((k_gemm_h3k<E, 2, 8, 2>), dim3((p.M + 63) / 64, (p.N + 63) / 64, gz), \
