@@ -132,7 +132,7 @@ struct GemmParams {
   // launch_gemm_h3 with GEMM_ADD: a buffer of kGemmPartsFloats.  Where
   // gemm_h3_splits(M, N, K) > 1 the partial sums of that many K ranges are
   // stored to parts[z][M][N] instead of being added to c, for the next
-  // launch_rows_rmsnorm to add.  Null: c is always complete.
+  // launch_rows_rmsnorm_planes (or launch_add_parts) to add.  Null: c is always complete.
   float* parts;
 };
 
@@ -172,12 +172,10 @@ struct FlashParams {
 hipError_t launch_gemm(const GemmParams& p, int epi, hipStream_t s);
 hipError_t launch_flash(const FlashParams& p, int batch, int max_rows,
                         hipStream_t s);
-// With nparts > 0 (size % 4 == 0, size <= kNormPartsMax) x first takes the
-// sum of the partial sums parts[z][rows][size]; out may then be null.
-constexpr int kNormPartsMax = 4096;
-hipError_t launch_rows_rmsnorm(float* x, const float* w, float* out, int rows, int size,
-                               float eps, hipStream_t s, const float* parts = nullptr,
-                               int nparts = 0);
+hipError_t launch_rows_rmsnorm(const float* x, const float* w, float* out,
+                               int rows, int size, float eps, hipStream_t s);
+// x[n] += the sum of the partial sums parts[z][n] (n % 4 == 0).
+hipError_t launch_add_parts(float* x, const float* parts, int nparts, size_t n, hipStream_t s);
 
 // The optional bfloat16-MFMA prefill: bfloat16 MFMA operands (round to
 // nearest even), fp32 accumulation, fp32 residual stream and KV cache.
@@ -204,8 +202,10 @@ int gemm_h3_splits(int M, int N, int K);
 size_t split_weights_f16_bytes(int K, int N);
 // The fp16 planes of `rows` rows of K floats, launch_gemm_h3's A, and the
 // producers that write them: the row norm (size % 8 == 0, size <=
-// kNormPartsMax), flash attention of these shapes (FlashParams::op16), GEMM_SILU
-// and a conversion of fp32 rows.
+// kNormPartsMax; with nparts > 0 x first takes the partial sums), flash
+// attention of these shapes (FlashParams::op16), GEMM_SILU and a conversion of
+// fp32 rows.
+constexpr int kNormPartsMax = 4096;
 size_t split_rows_f16_bytes(size_t rows, int K);
 hipError_t launch_rows_rmsnorm_planes(float* x, const float* w, uint16_t* planes, int rows,
                                       int size, float eps, hipStream_t s,

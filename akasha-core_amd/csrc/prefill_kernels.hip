@@ -30,22 +30,17 @@ __global__ void k_embedding_rows(const uint32_t* tokens, const float* table,
 // Rows of up to 4096 floats (a multiple of 4): one wave per row, four rows
 // per block, the row held in registers between the sum of squares (a wave
 // butterfly, no LDS or barrier) and the scaling, read and written 16 bytes
-// at a time.  PARTS (these sizes only): the row is first the sum of x and the
-// nparts partial sums of the GEMM before it (parts[z][row][:], added in order,
-// then to x), which is stored back to x; out may then be null for the sum
-// alone (an instantiation of its own: its registers would halve the waves of
-// the plain norm).  Other sizes: one block per row, element by element.
-template <int QL, bool PARTS = false>  // float4 per lane: size <= 256 QL
-__global__ __launch_bounds__(256) void k_rows_rmsnorm(float* __restrict__ x,
+// at a time.  Other sizes: one block per row, element by element.
+template <int QL>  // float4 per lane: size <= 256 QL
+__global__ __launch_bounds__(256) void k_rows_rmsnorm(const float* __restrict__ x,
                                                       const float* __restrict__ w,
                                                       float* __restrict__ out, int rows,
-                                                      int size, float eps,
-                                                      const float* __restrict__ parts,
-                                                      int nparts) {
+                                                      int size, float eps) {
   if (QL > 0) {
     const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (row >= rows) return;
-    float4* xr = reinterpret_cast<float4*>(x + (size_t)row * size);
+    const float4* xr = reinterpret_cast<const float4*>(x + (size_t)row * size);
+    float4* o = reinterpret_cast<float4*>(out + (size_t)row * size);
     const float4* g4 = reinterpret_cast<const float4*>(w);
     const int nq = size >> 2;
     float4 v[QL > 0 ? QL : 1], g[QL > 0 ? QL : 1];
@@ -54,42 +49,9 @@ __global__ __launch_bounds__(256) void k_rows_rmsnorm(float* __restrict__ x,
     for (int i = 0; i < QL; ++i) {
       const int q = lane + 64 * i;
       v[i] = q < nq ? xr[q] : make_float4(0.f, 0.f, 0.f, 0.f);
-      g[i] = out && q < nq ? g4[q] : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-    if (PARTS) {
-      constexpr int NB = QL <= 4 ? 4 : 2;  // partial sums per batch of loads
-      float4 sum[QL > 0 ? QL : 1];
-#pragma unroll
-      for (int i = 0; i < QL; ++i) sum[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-      for (int z = 0; z < nparts; z += NB) {
-        float4 t[NB][QL > 0 ? QL : 1];
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {
-          const float4* pr =
-              reinterpret_cast<const float4*>(parts + ((size_t)(z + b) * rows + row) * size);
-#pragma unroll
-          for (int i = 0; i < QL; ++i) {
-            const int q = lane + 64 * i;
-            t[b][i] = z + b < nparts && q < nq ? pr[q] : make_float4(0.f, 0.f, 0.f, 0.f);
-          }
-        }
-#pragma unroll
-        for (int b = 0; b < NB; ++b)
-#pragma unroll
-          for (int i = 0; i < QL; ++i) add4(sum[i], t[b][i]);
-      }
-#pragma unroll
-      for (int i = 0; i < QL; ++i) {
-        const int q = lane + 64 * i;
-        add4(v[i], sum[i]);
-        if (q < nq) xr[q] = v[i];
-      }
-      if (!out) return;
-    }
-    float4* o = reinterpret_cast<float4*>(out + (size_t)row * size);
-#pragma unroll
-    for (int i = 0; i < QL; ++i)
+      g[i] = q < nq ? g4[q] : make_float4(0.f, 0.f, 0.f, 0.f);
       ss += v[i].x * v[i].x + v[i].y * v[i].y + v[i].z * v[i].z + v[i].w * v[i].w;
+    }
     ss = wave_sum(ss);
     const float rs = 1.0f / sqrtf(ss / (float)size + eps);
 #pragma unroll
@@ -1697,6 +1659,18 @@ __global__ __launch_bounds__(512) void k_rows_rmsnorm_planes(float* __restrict__
   for (int q = threadIdx.x >> 3; q < 8 * steps; q += 64)  // q = 2 octet + plane
     reinterpret_cast<uint4*>(planes)[plane_piece(m, q >> 1, steps) + 64 * (q & 1)] =
         pieces[q * 9 + r];
+}
+
+// x += the sum of the nparts partial sums parts[z][n], in order (the last
+// ffn_down's, which no norm follows); n a multiple of 4.
+__global__ __launch_bounds__(256) void k_add_parts(float* __restrict__ x,
+                                                   const float* __restrict__ parts, int nparts,
+                                                   size_t n) {
+  const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i >= n) return;
+  float4 v = *reinterpret_cast<const float4*>(x + i);
+  add4(v, sum_parts4<8>(make_float4(0.f, 0.f, 0.f, 0.f), parts + i, n, nparts));
+  *reinterpret_cast<float4*>(x + i) = v;
 }
 
 // fp32 rows into A's planes, one 16-byte piece of each plane per thread (for
@@ -3315,29 +3289,24 @@ hipError_t launch_flash_bf16(const FlashParams& p, int batch, int max_rows, hipS
   return hipGetLastError();
 }
 
-hipError_t launch_rows_rmsnorm(float* x, const float* w, float* out, int rows, int size,
-                               float eps, hipStream_t s, const float* parts, int nparts) {
+hipError_t launch_rows_rmsnorm(const float* x, const float* w, float* out,
+                               int rows, int size, float eps, hipStream_t s) {
   const dim3 g((rows + 3) / 4);
-  if (nparts > 0 && (!parts || size % 4 != 0 || size > kNormPartsMax)) return hipErrorInvalidValue;
-  if (nparts <= 0 && !out) return hipErrorInvalidValue;
-#define AKH_NORM_GO(QL)                                                                          \
-  if (nparts > 0)                                                                                \
-    hipLaunchKernelGGL((k_rows_rmsnorm<QL, true>), g, dim3(256), 0, s, x, w, out, rows, size,     \
-                       eps, parts, nparts);                                                      \
-  else                                                                                           \
-    hipLaunchKernelGGL((k_rows_rmsnorm<QL>), g, dim3(256), 0, s, x, w, out, rows, size, eps,      \
-                       nullptr, 0);
-  if (size % 4 != 0 || size > kNormPartsMax) {
-    hipLaunchKernelGGL(k_rows_rmsnorm<0>, dim3(rows), dim3(256), 0, s, x, w, out, rows, size, eps,
-                       nullptr, 0);
-  } else if (size <= 1024) {
-    AKH_NORM_GO(4)
-  } else if (size <= 2048) {
-    AKH_NORM_GO(8)
-  } else {
-    AKH_NORM_GO(16)
-  }
-#undef AKH_NORM_GO
+  if (size % 4 != 0 || size > 4096)
+    hipLaunchKernelGGL(k_rows_rmsnorm<0>, dim3(rows), dim3(256), 0, s, x, w, out, rows, size, eps);
+  else if (size <= 1024)
+    hipLaunchKernelGGL(k_rows_rmsnorm<4>, g, dim3(256), 0, s, x, w, out, rows, size, eps);
+  else if (size <= 2048)
+    hipLaunchKernelGGL(k_rows_rmsnorm<8>, g, dim3(256), 0, s, x, w, out, rows, size, eps);
+  else
+    hipLaunchKernelGGL(k_rows_rmsnorm<16>, g, dim3(256), 0, s, x, w, out, rows, size, eps);
+  return hipGetLastError();
+}
+
+hipError_t launch_add_parts(float* x, const float* parts, int nparts, size_t n, hipStream_t s) {
+  if (!x || !parts || nparts <= 0 || n == 0 || n % 4 != 0) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_add_parts, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, s, x, parts,
+                     nparts, n);
   return hipGetLastError();
 }
 

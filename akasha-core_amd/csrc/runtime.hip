@@ -2077,7 +2077,7 @@ hipError_t prefill_norm(akh_session* s, const float* gain, size_t rows, bool pla
     return launch_rows_rmsnorm_planes(s->px, gain, xn16, (int)rows, d, eps, st, s->pparts,
                                       pending);
   if (!planes)
-    return launch_rows_rmsnorm(s->px, gain, s->pxn, (int)rows, d, eps, st, s->pparts, pending);
+    return launch_rows_rmsnorm(s->px, gain, s->pxn, (int)rows, d, eps, st);
   // Rows wider than the norm's registers: fp32 rows first.
   hipError_t e = launch_rows_rmsnorm(s->px, gain, s->pwide, (int)rows, d, eps, st);
   return e == hipSuccess ? launch_rows_planes(s->pwide, (int)rows, d, xn16, st) : e;
@@ -2200,8 +2200,7 @@ hipError_t prefill_layers_f32(akh_session* s, const PrefillRows& pr, bool exact)
     TRY_HIP(add_gemm(w, base + W_DOWN));
   }
   if (pending > 0)  // the last ffn_down's, with no norm: px alone
-    TRY_HIP(launch_rows_rmsnorm(s->px, nullptr, nullptr, (int)rows, (int)d, c.norm_eps, st,
-                                s->pparts, pending));
+    TRY_HIP(launch_add_parts(s->px, s->pparts, pending, rows * d, st));
 #undef TRY_HIP
   return hipSuccess;
 }
