@@ -829,6 +829,10 @@ __device__ __forceinline__ uint32_t pick_binned(const SampleArgs& a, int m, int 
     bad |= rh.head[q].bad;
   }
   if (bad || mx == -INFINITY) return none;  // uniform
+  // Cells are whole floats: every one from the row's first bin to the one past
+  // its last has to be exact, or a bin's edge (cell - b below) rounds onto its
+  // neighbour's and the bin's members are lost.
+  if (!(fabsf(grid_cell(mx, scale)) + (float)(kCells + 1) <= 0x1p24f)) return none;
   const double mxd = (double)mx, T = (double)a.temperature;
   if (t < parts)
     rh.part_f[t] = rh.head[t].max == -INFINITY ? 0.0 : exp(((double)rh.head[t].max - mxd) / T);
@@ -967,12 +971,15 @@ __device__ __forceinline__ uint32_t pick_binned(const SampleArgs& a, int m, int 
     __syncthreads();
     total = rh.target;
   }
+  // The walk stops in its own bins: the entries of a cut bin below them are
+  // not what follows them in the order.
   const double stop = r * total;
   const uint32_t pick = first_entry([&](int e, double thru) {
-    return (uint32_t)(2 * t + e) <= cut && thru > stop;
+    return (uint32_t)(2 * t + e) <= cut && be[e] <= w1 && thru > stop;
   });
-  // No entry passes (r * total rounded up to total): the last kept one.
-  if (pick == 0xFFFFFFFFu) return cutting ? index_of(cut) : none;
+  // No entry passes: the last kept one where r * total rounded up to total,
+  // else the bins' sums and the entries' differ by a rounding at w1's end.
+  if (pick == 0xFFFFFFFFu) return cutting && c == w1 ? index_of(cut) : none;
   return index_of(pick);
 }
 

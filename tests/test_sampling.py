@@ -183,3 +183,25 @@ def test_device_sampler_binned_rows(backend, pkg, ora, rows, n, t, k, p):
     check = range(rows) if rows < 10 else list(range(8)) + [rows - 1]
     want = [ora.sample_token(l[i], t, k, p, seen_rows[i], 1.15, u[i]) for i in check]
     assert [int(got[i]) for i in check] == want
+
+
+# Binned rows whose grid cells (64 per logit, or 48 per unit of logit /
+# temperature) lie below, across and above 2^24, where floats stop holding
+# every whole number: large logits of both signs, and small temperatures.
+@pytest.mark.gpu
+@pytest.mark.parametrize("mean,std,t,p", [
+    (2.6e5, 2.0, 0.8, 0.95), (-2.6e5, 2.0, 0.8, 0.5), (262140.0, 3.0, 0.8, 0.95),
+    (262140.0, 3.0, 0.8, 0.5), (-262144.0, 3.0, 0.8, 0.5), (3e5, 2.0, 0.8, 0.95),
+    (-3e5, 2.0, 0.8, 0.9), (400.0, 0.002, 1e-3, 0.95), (50.0, 0.001, 1e-4, 0.95),
+    (50.0, 0.001, 1e-4, 0.5), (6.0, 1e-4, 1e-5, 0.95), (4500.0, 1.0, 0.01, 0.9),
+    (262140.0, 3.0, 0.8, 1.0),
+])
+def test_device_sampler_binned_rows_far_cells(backend, pkg, ora, mean, std, t, p):
+    rows, n = 200, 5000
+    for seed in (1, 2, 3):
+        rng = np.random.default_rng(seed)
+        l = (mean + std * rng.standard_normal(n)).astype(np.float32)
+        u = rng.random(rows)
+        got = _device_sample(pkg, backend, np.tile(l, (rows, 1)), t, 0, p, 1.0, [[]] * rows, u)
+        want = [ora.sample_token(l, t, 0, p, [], 1.0, x) for x in u]
+        assert list(got) == want, seed
