@@ -59,15 +59,37 @@ constexpr int NW = NT / 64;     // waves per block
 
 // Radix digits of the order keys: 11, 11 and 10 bits (three passes).
 constexpr int kBins = 2048;
+constexpr int kPartsMax = 16;  // of a binned row (below)
+struct PartHead {
+  float max;
+  int bad;       // NaN, an infinite maximum, a grid beyond 2^30
+  double total;  // of the part's weights (or its count)
+};
+struct RowHist {
+  double before[kBins];  // weight (or count) of the bins above
+  PartHead head[kPartsMax];
+  double part_f[kPartsMax];
+  uint32_t first[2];     // list position of a run's first entry
+  double target;
+};
+// A block's LDS also holds the seen-id bitmap (an eighth of a byte per id), so
+// what never lives together shares its place: a binned row's totals and the
+// radix path's bins here, the list before and after its sort in TopKShared.
+// Together 58.7 KB: vocabularies of up to 840 thousand ids with a penalty.
 struct SampleShared {
-  // One radix pass's bins: counts or f64 weight sums (a select uses one).
   union {
-    uint32_t hist_n[kBins];
-    double hist_w[kBins];
+    struct {
+      // One radix pass's bins: counts or f64 weight sums (a select uses one).
+      union {
+        uint32_t hist_n[kBins];
+        double hist_w[kBins];
+      };
+      // The last pass's bins (kBins / 2): members of nonzero weight, lowest index.
+      uint32_t last_n[kBins / 2];
+      uint32_t last_i[kBins / 2];
+    };
+    RowHist rh;
   };
-  // The last pass's bins (kBins / 2): members of nonzero weight, lowest index.
-  uint32_t last_n[kBins / 2];
-  uint32_t last_i[kBins / 2];
   double wave_d[NW];
   uint32_t wave_u[NW];
   float wave_f[NW];
@@ -266,7 +288,10 @@ constexpr int CCAP = 2048;  // candidates gathered for the sort
 constexpr int NTH = 16;     // thresholds counted per pass
 
 struct TopKShared {
-  unsigned long long comp[CCAP];  // key << 32 | ~index: descending = the order
+  union {
+    unsigned long long comp[CCAP];  // key << 32 | ~index: descending = the order
+    double pre[CCAP];               // once sorted: weight of the entries before each
+  };
   union {
     struct {
       unsigned long long top[KCAP];  // the first entries of that order
@@ -699,13 +724,9 @@ __device__ __forceinline__ bool row_seen(const SampleArgs& a, int m, SeenIds& s)
 // every id up again.
 // ---------------------------------------------------------------------------
 constexpr int kCells = kBins - 1;
-constexpr int kPartsMax = 16;
-struct PartHead {
-  float max;
-  int bad;       // NaN, an infinite maximum, a grid beyond 2^30
-  double total;  // of the part's weights (or its count)
-};
 static_assert(sizeof(PartHead) == 2 * sizeof(double), "two doubles of the row's workspace");
+static_assert(sizeof(SampleShared) + sizeof(TopKShared) + 840000 / 8 <= 160 * 1024,
+              "a block's LDS beside the bitmap of 840000 ids");
 static_assert(kBins == 2 * NT && CCAP == 2 * NT, "two bins and two list entries per thread");
 // Doubles of the workspace before the penalised logits.
 __host__ __device__ constexpr long hist_doubles(int parts) { return (long)parts * (kBins + 2); }
@@ -800,20 +821,12 @@ __global__ __launch_bounds__(NT) void k_sample_hist(SampleArgs a) {
     reinterpret_cast<PartHead*>(base + (size_t)parts * kBins)[part] = PartHead{mx, bad, total};
 }
 
-struct RowHist {
-  double before[kBins];  // weight (or count) of the bins above
-  PartHead head[kPartsMax];
-  double part_f[kPartsMax];
-  uint32_t first[2];     // list position of a run's first entry
-  double pre[CCAP];      // weight of the list's entries before each
-  double target;
-};
-
 // The pick of row m from its parts' bins, or n where the radix path must
 // decide.  Every thread of the block calls it.
 __device__ __forceinline__ uint32_t pick_binned(const SampleArgs& a, int m, int parts,
-                                                const float* src, double r, SampleShared& sh, TopKShared& tk,
-                                                RowHist& rh) {
+                                                const float* src, double r, SampleShared& sh,
+                                                TopKShared& tk) {
+  RowHist& rh = sh.rh;
   const uint32_t none = (uint32_t)a.n;
   const int n = a.n, t = threadIdx.x;
   const bool count = a.top_k > 0 && a.top_k < n;
@@ -941,14 +954,14 @@ __device__ __forceinline__ uint32_t pick_binned(const SampleArgs& a, int m, int 
     }
   }
   const double pre = block_scan_excl<double>(we[0] + we[1], sh.wave_d);
-  if (2 * t < nc) rh.pre[2 * t] = pre;
-  if (2 * t + 1 < nc) rh.pre[2 * t + 1] = pre + we[0];
+  if (2 * t < nc) tk.pre[2 * t] = pre;
+  if (2 * t + 1 < nc) tk.pre[2 * t + 1] = pre + we[0];
   __syncthreads();
   // The row's running total through entry k.
   auto through = [&](int e) {
     const int k = 2 * t + e;
     const bool low = be[e] > w1;
-    return rh.before[low ? c : w0] + ((rh.pre[k] - rh.pre[rh.first[low ? 1 : 0]]) + we[e]);
+    return rh.before[low ? c : w0] + ((tk.pre[k] - tk.pre[rh.first[low ? 1 : 0]]) + we[e]);
   };
   auto first_entry = [&](auto test) {
     uint32_t mine = 0xFFFFFFFFu;
@@ -988,7 +1001,6 @@ __global__ __launch_bounds__(NT) void k_sample_rows(SampleArgs a, int parts) {
   extern __shared__ uint32_t bitmap[];
   __shared__ SampleShared sh;
   __shared__ TopKShared tk;
-  __shared__ RowHist rh;
   const int m = blockIdx.x, n = a.n;
   const float* row = a.logits + (size_t)m * a.row_stride;
   double* w = a.wbuf + (size_t)m * n;
@@ -1005,7 +1017,7 @@ __global__ __launch_bounds__(NT) void k_sample_rows(SampleArgs a, int parts) {
     const float* src = a.penalty == 1.0f || !seen.ids
                            ? row
                            : reinterpret_cast<const float*>(w + hist_doubles(parts));
-    pick = pick_binned(a, m, parts, src, r, sh, tk, rh);
+    pick = pick_binned(a, m, parts, src, r, sh, tk);
     __syncthreads();  // the other paths reuse the row's workspace and LDS
   }
   const uint32_t* bm = pick < (uint32_t)n ? nullptr : seen_bitmap(a, seen, bitmap);

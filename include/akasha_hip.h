@@ -238,7 +238,8 @@ typedef struct {
  * [rows, seen_stride] with seen_len[rows] valid entries (NULL: no seen ids);
  * uniforms may be NULL when temperature <= 0.  Ids with equal logits are
  * ordered lower index first (the reference's unstable sort leaves that
- * order unspecified).  n <= 2^20. */
+ * order unspecified).  n <= 2^20, and with a repetition penalty over seen
+ * ids n <= 840000 (their bitmap shares a block's LDS; AKH_E_HIP beyond). */
 akh_status akh_sample_rows(akh_backend* be, const float* logits, uint32_t rows,
                            uint32_t n, akh_sampling params, const uint32_t* seen,
                            uint32_t seen_stride, const uint32_t* seen_len,

@@ -205,3 +205,19 @@ def test_device_sampler_binned_rows_far_cells(backend, pkg, ora, mean, std, t, p
         got = _device_sample(pkg, backend, np.tile(l, (rows, 1)), t, 0, p, 1.0, [[]] * rows, u)
         want = [ora.sample_token(l, t, 0, p, [], 1.0, x) for x in u]
         assert list(got) == want, seed
+
+
+# The largest vocabulary with a penalty: its bitmap takes the LDS that the
+# sampler's own arrays leave.  Greedy, binned and radix rows.
+@pytest.mark.gpu
+@pytest.mark.parametrize("t,k,p", [(0.0, 0, 1.0), (0.7, 40, 0.95), (0.7, 0, 0.9), (0.7, 3000, 0.9)])
+def test_device_sampler_largest_vocabulary_with_penalty(backend, pkg, ora, t, k, p):
+    rows, n = 2, 840000
+    rng = np.random.default_rng(5)
+    l = (rng.standard_normal((rows, n)) * 2.5).astype(np.float32)
+    top = np.argsort(-l, axis=1)[:, :8]
+    seen_rows = [np.append(top[i], n - 1).astype(np.uint32) for i in range(rows)]
+    u = rng.random(rows)
+    got = _device_sample(pkg, backend, l, t, k, p, 1.3, seen_rows, u)
+    want = [ora.sample_token(l[i], t, k, p, seen_rows[i], 1.3, u[i]) for i in range(rows)]
+    assert list(got) == want
