@@ -2131,6 +2131,20 @@ int dec_few_splits(int K, int N) {
   return std::max(1, std::min({AKH_FEW_BLOCKS / tiles, K / AKH_FEW_KMIN, kFewParts}));
 }
 
+// ffn_down's blocks are the ones with the longest range of K (`per` k-quads),
+// and they hold it in LDS per row; a wide row adds to what every block
+// computes again.  Both grow with the rows, where the batched kernels' MFMAs
+// do not.  us per step of 4 layers on MI355X, batched / here: one and two rows,
+// dim 512 ffn 8192 (per 171) 140 / 125 and 155 / 142, dim 1024 ffn 6144 (192) 157 /
+// 174 and 179 / 192, dim 32 ffn 65536 (1366) 176 / 378; three, dim 256 ffn 8192
+// (171) 137 / 132, dim 768 ffn 6144 (154) 160 / 166; four, dim 1024 ffn 3072 (96)
+// 164 / 159, ffn 4096 (128) 170 / 173, dim 256 ffn 8192 (171) 137 / 145.
+bool dec_few_pays(int M, int dim, int ffn) {
+  const int splits = dec_few_splits(ffn, dim), per = (ffn / 4 + splits - 1) / splits;
+  return M >= 1 && M <= kDecFewRows && dim <= kDecFewMaxK &&
+         24l * per + dim <= 6700 - 750 * std::max(M, 2);
+}
+
 hipError_t launch_dec_few(const DecFewParams& p, int pro, hipStream_t s) {
   if (p.M < 1 || p.M > kDecFewRows || p.K % 4 != 0 || p.K <= 0 || (p.w && p.splits < 1) ||
       (pro == FEW_NORM && p.K > kDecFewMaxK) || (pro != FEW_NORM && !p.w))
@@ -2138,6 +2152,7 @@ hipError_t launch_dec_few(const DecFewParams& p, int pro, hipStream_t s) {
   const int nq = p.K / 4, per = p.w ? (nq + p.splits - 1) / p.splits : 0;
   const dim3 g(p.w ? (p.N + 31) / 32 : 1, p.w ? p.splits : 1);
   const size_t lds = (size_t)p.M * (pro == FEW_NORM ? nq : per) * sizeof(float4);
+  if (lds > 60 * 1024) return hipErrorInvalidValue;  // beside the block's static 2 KB
 #define AKH_FEW_NI(PRO, M)                                               \
   if (per <= 32)                                                         \
     hipLaunchKernelGGL((k_dec_few<PRO, M, 4>), g, dim3(256), lds, s, p);  \

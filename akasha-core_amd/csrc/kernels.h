@@ -436,6 +436,7 @@ constexpr int kDecFewRows = 4;     // most sequences
 constexpr int kDecFewMaxK = 1024;  // widest row a block norms
 constexpr int kFewParts = 12;      // most splits, whose sums load at once
 int dec_few_splits(int K, int N);
+bool dec_few_pays(int M, int dim, int ffn);  // against the batched kernels
 hipError_t launch_dec_few(const DecFewParams& p, int pro, hipStream_t s);
 
 // Per-row residual update + RMSNorm: x = table[ids[m]] (zero row if the id

@@ -1910,7 +1910,7 @@ akh_status session_create(akh_model* m, uint32_t max_context_len, uint32_t batch
   alloc((void**)&s->p_up, (size_t)s->ks_up * R * F * 4);
   if (silu_own_kernel(s)) alloc((void**)&s->up_act, R * F * 4);
   alloc((void**)&s->p_down, (size_t)s->ks_down * R * d * 4);
-  if (batch <= (uint32_t)kDecFewRows && d <= (size_t)kDecFewMaxK) {
+  if (batch <= (uint32_t)kDecFewRows && dec_few_pays((int)batch, (int)d, (int)F)) {
     // k_dec_few's residual rows (two versions) and partial sums.
     const size_t M = batch;
     auto parts = [](size_t K, size_t N) { return (size_t)dec_few_splits((int)K, (int)N) * N; };

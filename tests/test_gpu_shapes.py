@@ -194,3 +194,29 @@ def test_few_sequences_decode_matches_oracle(backend, pkg, ora, batch, dim, head
     s.truncate(3)
     assert np.array_equal(greedy, np.stack([s.decode_step(None)[1] for _ in range(9)]))
     s.close()
+
+
+# Feed-forwards too long for those GEMVs decode on the batched kernels, with the
+# sequences at which that begins: the last that one to three take, the first
+# that none takes, one whose rows would not fit a block's LDS.
+@pytest.mark.parametrize("batch,dim,ffn,few", [
+    (3, 32, 8192, True), (4, 32, 8192, False), (1, 64, 12288, False), (4, 32, 131072, False),
+])
+def test_few_sequences_long_ffn_matches_oracle(backend, pkg, ora, batch, dim, ffn, few):
+    cfg = dataclasses.replace(pkg.ModelConfig.new(173, dim, 2, 2, 24), ffn_hidden=ffn)
+    w = pkg.synthetic_weights(cfg, seed=93, std=0.02)
+    model = pkg.hip.Model(backend, cfg)
+    model.upload(w)
+    s = pkg.hip.Session(model, 24, batch)
+    assert s.decode_launches() == (5 * 2 + 3 if few else 7 * 2 + 3)
+    prompts = [pkg.synthetic_tokens(3 + 2 * b, 173, seed=94 + b) for b in range(batch)]
+    logits, nxt = s.prefill(prompts)
+    refs = [ora.OracleSession(cfg, w, 24) for _ in range(batch)]
+    want = [r.prefill(p) for r, p in zip(refs, prompts)]
+    for step in range(3):
+        for b in range(batch):
+            assert np.abs(logits[b] - want[b]).max() < 1e-3, (step, b)
+            assert int(nxt[b]) == ora.argmax(want[b]), (step, b)
+        want = [r.decode_step(int(t)) for r, t in zip(refs, nxt)]
+        logits, nxt = s.decode_step(None)
+    s.close()
