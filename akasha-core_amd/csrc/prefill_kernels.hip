@@ -1310,6 +1310,8 @@ __global__ __launch_bounds__(64 * WM * WN * KG, 2) void k_gemm_h3(GemmParams p) 
           is_a ? ((uint32_t)min(f >> 2, rt_last) * steps + step) * 4096u + (f & 3) * 1024u
                : ((uint32_t)min(f >> 3, cg_last) * steps + step) * 8192u + (f & 7) * 1024u;
       const uint32_t dst = base + buf * STAGE + c * 1024;
+      // m0 is a reserved register, which a clobber list must not name; nothing
+      // else in the kernel reads it (no other LDS DMA, message or indexed move).
       asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                    :
                    : "s"(dst), "v"(vo), "s"(is_a ? rsa : rsb), "s"(so)
@@ -1366,12 +1368,12 @@ __global__ __launch_bounds__(64 * WM * WN * KG, 2) void k_gemm_h3(GemmParams p) 
   int buf = 0;
   for (int it = 0; it < iters; ++it) {
     // This step's pieces have landed; with three buffers the next step's may
-    // still be in flight.
+    // still be in flight.  Wait and barrier are one statement that clobbers
+    // memory (the barrier's builtin does not), so no LDS read moves before it.
     if (ST > 2 && step_of(it + 1) < s1)
-      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(CH) : "memory");
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(CH) : "memory");
     else
-      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" : : : "memory");
-    __builtin_amdgcn_s_barrier();
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" : : : "memory");
     const int nbuf = buf == 0 ? ST - 1 : buf - 1;  // the buffer of step it - 1
     if (step_of(it + ST - 1) < s1) issue(step_of(it + ST - 1), nbuf);
     if (KG == 1 || step_of(it) < s1) compute(buf);
