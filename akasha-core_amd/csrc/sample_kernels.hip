@@ -62,7 +62,7 @@ constexpr int kBins = 2048;
 constexpr int kPartsMax = 16;  // of a binned row (below)
 struct PartHead {
   float max;
-  int bad;       // NaN, an infinite maximum, a grid beyond 2^30
+  float scale;   // of the row's grid; 0: NaN or an infinite maximum in the part
   double total;  // of the part's weights (or its count)
 };
 struct RowHist {
@@ -734,11 +734,19 @@ __host__ __device__ constexpr long hist_doubles(int parts) { return (long)parts 
 // an id, of the workspace's 8).
 constexpr int kHistMin = 2 * (kBins + 2);
 
-// About 64 cells per logit or 48 per unit of l / T, whichever is finer: cells
-// of ~150 ids at the densest of 50257 logits N(0, 2^2), and 2047 cells reach
-// 42 T below the maximum (e^-42 of its weight) or 32.
-__device__ __forceinline__ float grid_scale(float temperature) {
-  return fmaxf(64.0f, 48.0f / temperature);
+// Cells per logit: 64, or 48 per unit of l / T where that is finer (cells of
+// ~150 ids at the densest of 50257 logits N(0, 2^2); 2047 cells reach 42 T below
+// the maximum, e^-42 of its weight, or 32), or finer still on a flat row,
+// whose logits would share a few cells: 800 to the range lo .. hi of 1024 of the
+// row's logits, which is about 6.5 standard deviations (32 rows x 50257 N(0,
+// 0.01^2) on MI355X, us without / with: top_k 40 108 / 23, top_p alone 173 / 36).
+// No finer than keeps hi's cell at 2^23, so that a large maximum's cells are
+// exact (far below zero hi is a mask's value and says nothing of the maximum).
+__device__ __forceinline__ float grid_scale(float temperature, float hi, float lo) {
+  float s = fmaxf(64.0f, 48.0f / temperature);
+  if (hi > lo) s = fmaxf(s, 800.0f / (hi - lo));
+  if (hi > -1e4f && hi < INFINITY) s = fminf(s, 0x1p23f / fabsf(hi));
+  return fminf(s, 0x1p60f);
 }
 __device__ __forceinline__ float grid_cell(float l, float scale) {
   return floorf(__fmul_rn(l, scale));
@@ -756,6 +764,9 @@ __global__ __launch_bounds__(NT) void k_sample_hist(SampleArgs a) {
   const int per = (a.n + parts - 1) / parts, lo = min(a.n, part * per);
   const int len = min(a.n, lo + per) - lo;
   auto l_at = [&](int i) { return pen_logit(row, lo + i, bm, a.penalty); };
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  // The same 1024 logits of the row for each of its parts, for their grid.
+  const float some = row[(long)(a.n - 64) * wave / (NW - 1) + lane];
   // A part of up to NT * U ids stays in registers between the two passes.
   float v[U];
 #pragma unroll
@@ -779,20 +790,38 @@ __global__ __launch_bounds__(NT) void k_sample_hist(SampleArgs a) {
     for (int i = U * NT + (int)threadIdx.x; i < len; i += NT) copy[i] = l_at(i);
   }
   float mxv = -INFINITY;
-  uint32_t nan = 0;
+  bool nan = false;
   each([&](float l) {
-    if (l != l) nan = 1;
-    else mxv = fmaxf(mxv, l);
+    nan = nan || l != l;
+    mxv = fmaxf(mxv, l);
   });
   for (int b = threadIdx.x; b < kBins; b += NT) {
     if (count) sh.hist_n[b] = 0u;
     else sh.hist_w[b] = 0.0;
   }
-  const float mx = block_max_f(mxv, sh);
-  const float scale = grid_scale(a.temperature);
-  const bool empty = mx == -INFINITY;
-  const bool bad = __syncthreads_or((int)nan) || mx == INFINITY ||
-                   (!empty && !(fabsf(mx) * scale < 0x1p30f));
+  // The part's maximum, the range of `some` and whether there is a NaN.
+  {
+    const bool any_nan = __any(nan);
+    const float x = wave_max(mxv), top = wave_max(some), neg = wave_max(-some);
+    if (lane == 0) {
+      sh.wave_f[wave] = x;
+      reinterpret_cast<float2*>(sh.wave_d)[wave] = make_float2(top, neg);
+      sh.wave_u[wave] = any_nan;
+    }
+  }
+  __syncthreads();
+  float mx = -INFINITY, hi = -INFINITY, nlo = -INFINITY;
+  uint32_t nans = 0;
+#pragma unroll
+  for (int k = 0; k < NW; ++k) {
+    const float2 r = reinterpret_cast<const float2*>(sh.wave_d)[k];
+    mx = fmaxf(mx, sh.wave_f[k]);
+    hi = fmaxf(hi, r.x);
+    nlo = fmaxf(nlo, r.y);
+    nans |= sh.wave_u[k];
+  }
+  const float scale = grid_scale(a.temperature, hi, -nlo);
+  const bool empty = mx == -INFINITY, bad = nans || mx == INFINITY;
   double own = 0.0;
   if (!bad && !empty) {
     const float cell = grid_cell(mx, scale);
@@ -818,7 +847,8 @@ __global__ __launch_bounds__(NT) void k_sample_hist(SampleArgs a) {
     }
   }
   if (threadIdx.x == 0)
-    reinterpret_cast<PartHead*>(base + (size_t)parts * kBins)[part] = PartHead{mx, bad, total};
+    reinterpret_cast<PartHead*>(base + (size_t)parts * kBins)[part] =
+        PartHead{mx, bad ? 0.f : scale, total};
 }
 
 // The pick of row m from its parts' bins, or n where the radix path must
@@ -830,22 +860,22 @@ __device__ __forceinline__ uint32_t pick_binned(const SampleArgs& a, int m, int 
   const uint32_t none = (uint32_t)a.n;
   const int n = a.n, t = threadIdx.x;
   const bool count = a.top_k > 0 && a.top_k < n;
-  const float scale = grid_scale(a.temperature);
   const double* base = a.wbuf + (size_t)m * n;
   const PartHead* head = reinterpret_cast<const PartHead*>(base + (size_t)parts * kBins);
   if (t < parts) rh.head[t] = head[t];
   __syncthreads();
-  float mx = -INFINITY;
-  int bad = 0;
+  float mx = -INFINITY, scale = INFINITY;
   for (int q = 0; q < parts; ++q) {
     mx = fmaxf(mx, rh.head[q].max);
-    bad |= rh.head[q].bad;
+    scale = fminf(scale, rh.head[q].scale);  // one value, or 0 of a part
   }
-  if (bad || mx == -INFINITY) return none;  // uniform
+  if (scale == 0.f || mx == -INFINITY) return none;  // uniform
   // Cells are whole floats: every one from the row's first bin to the one past
   // its last has to be exact, or a bin's edge (cell - b below) rounds onto its
-  // neighbour's and the bin's members are lost.
-  if (!(fabsf(grid_cell(mx, scale)) + (float)(kCells + 1) <= 0x1p24f)) return none;
+  // neighbour's and the bin's members are lost.  The one edge that a count's
+  // cut takes is some logit's own cell, exact wherever cells are finite.
+  const float cell = grid_cell(mx, scale);
+  if (!(fabsf(cell) <= (count ? 0x1p30f : 0x1p24f - (float)(kCells + 1)))) return none;
   const double mxd = (double)mx, T = (double)a.temperature;
   if (t < parts)
     rh.part_f[t] = rh.head[t].max == -INFINITY ? 0.0 : exp(((double)rh.head[t].max - mxd) / T);
@@ -855,7 +885,6 @@ __device__ __forceinline__ uint32_t pick_binned(const SampleArgs& a, int m, int 
 
   // Thread t's bins 2 t and 2 t + 1 over the parts, then every bin's total
   // above it.
-  const float cell = grid_cell(mx, scale);
   // Eight parts' loads at a time, without branches between them (a part past
   // the last, an empty one and bins outside a part read bin 0 and count 0).
   double v[2] = {0.0, 0.0};

@@ -221,3 +221,33 @@ def test_device_sampler_largest_vocabulary_with_penalty(backend, pkg, ora, t, k,
     got = _device_sample(pkg, backend, l, t, k, p, 1.3, seen_rows, u)
     want = [ora.sample_token(l[i], t, k, p, seen_rows[i], 1.3, u[i]) for i in range(rows)]
     assert list(got) == want
+
+
+# Binned rows whose grid follows their logits: flat ones (down to a range of a
+# few floats, and all equal), half of the ids or all but eight at a mask's value,
+# a grid capped by large logits, and the same 1024 ids being all masked.
+@pytest.mark.gpu
+@pytest.mark.parametrize("t,k,p", [(0.8, 40, 0.95), (0.8, 0, 0.95), (1.0, 0, 1.0), (1e-4, 40, 0.9),
+                                   (1e-4, 0, 0.9), (0.7, 1000, 0.99)])
+def test_device_sampler_binned_rows_flat_and_masked(backend, pkg, ora, t, k, p):
+    rows, n = 12, 20003
+    rng = np.random.default_rng(11)
+    g = rng.standard_normal((rows, n))
+    l = (g * 2.5).astype(np.float32)
+    l[0] = g[0] * 0.01
+    l[1] = 30 + g[1] * 1e-3
+    l[2] = 1 + g[2] * 1e-6
+    l[3] = -7.5
+    l[4, n // 2:] = -1e30
+    l[5] = np.where(rng.permutation(n) < 8, l[5], np.float32(-1e30))
+    l[6] = np.where(rng.permutation(n) < 8, l[6], np.float32(-np.inf))
+    l[7, : n // 3] = -65504.0
+    l[8] = g[8] * 1e5
+    l[9] = 1e8 + g[9] * 100
+    l[10] = np.float32(1e-42) * np.round(g[10])
+    u = rng.random(rows)
+    seen_rows = [rng.integers(0, n, 40).astype(np.uint32) for _ in range(rows)]
+    for pen in (1.0, 1.15):
+        got = _device_sample(pkg, backend, l, t, k, p, pen, seen_rows, u)
+        want = [ora.sample_token(l[i], t, k, p, seen_rows[i], pen, u[i]) for i in range(rows)]
+        assert list(got) == want, pen
