@@ -1207,12 +1207,27 @@ hipError_t launch_sample_rows(const SampleArgs& a, int rows, hipStream_t s) {
     return hipErrorInvalidValue;
   const size_t lds = a.penalty != 1.0f && (a.seen || a.tok) ? (size_t)(a.n + 31) / 32 * 4 : 0;
   // Sampled rows long enough for at least one part's bins in their workspace of
-  // n doubles (top_k above KCAP stays on the radix path): about 256 blocks of
-  // bins in all, at most 16 parts a row (us for 32 x 50257 on MI355X, one block
-  // per row / binned: top_p alone 164 / 32.6, top_k 40 with top_p 36.8 / 28.8).
+  // n doubles (top_k above KCAP stays on the radix path).  us on MI355X, one block
+  // per row / binned: 32 x 50257 top_p alone 142 / 32.6, top_k 40 with top_p 37.9
+  // / 28.6; 1 x 4100 29.6 / 23.3 and 34.5 / 21.9.
+  // With temperature alone the radix path runs one select instead of two, and
+  // short rows stay there: 32 x 8000 23.0 / 23.7, 32 x 8200 (two parts) 23.5 / 22.9,
+  // 256 x 7000 23.9 / 25.4, 256 x 8000 28.3 / 25.7; over one row per CU 320 x 5000 37.8 / 40.6,
+  // 512 x 6000 46.4 / 43.6, 1024 x 4100 78 / 78.
+  const bool cut = a.top_p < 1.0f || (a.top_k > 0 && a.top_k < a.n);
+  const int from = cut || rows > 768 ? kHistMin
+                   : rows > 256      ? 5500
+                   : rows > 128      ? 7800
+                                     : 2 * kHistMin;
   int parts = 0;
-  if (a.temperature > 0.0f && a.n >= kHistMin && (a.top_k <= KCAP || a.top_k >= a.n)) {
-    parts = std::min(kPartsMax, std::max(1, AKH_SAMPLE_BLOCKS / rows));
+  if (a.temperature > 0.0f && a.n >= from && (a.top_k <= KCAP || a.top_k >= a.n)) {
+    // Parts for about 256 blocks of bins in all, at most 16 a row, and no part
+    // above 32768 ids while there are at most 1024 blocks (top_k 40 with top_p and
+    // a penalty, us at 1, 2, 4 and 8 parts: 256 x 131072 236, 169, 157, 144; 256 x
+    // 50257 79, 62, 58, 67; 512 x 131072 337, 315, 315, 296, top_p alone 294, 289,
+    // 291, 310).
+    parts = std::max(AKH_SAMPLE_BLOCKS / rows, std::min((a.n + 32767) / 32768, 1024 / rows));
+    parts = std::min(kPartsMax, std::max(1, parts));
     while (parts > 1 && (2 * hist_doubles(parts) > a.n || a.n / parts < NT)) --parts;
     hipLaunchKernelGGL(k_sample_hist, dim3(rows, parts), dim3(NT), lds, s, a);
   }
