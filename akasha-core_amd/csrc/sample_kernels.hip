@@ -51,9 +51,6 @@ namespace {
 #ifndef AKH_SAMPLE_BLOCKS
 #define AKH_SAMPLE_BLOCKS 256
 #endif
-#ifndef AKH_GATHER_U
-#define AKH_GATHER_U 25
-#endif
 constexpr int NT = AKH_SAMPLE_NT;  // threads per row (per part of a binned row)
 constexpr int NW = NT / 64;     // waves per block
 
@@ -514,17 +511,24 @@ __device__ __forceinline__ float cell_low(float cell, float scale) {
 // bit per id, and the few that are set are appended in a loop: a dispatch
 // starts with cold instruction caches, and straight-line code for every id of
 // a chunk cost more to fetch than to run (the row kernel on 32 x 50257: 25 us
-// so, 21 here; 25 ids a thread, two rounds of loads, against 16: 1 to 2 us).
+// so, 21 here).  Loads past the row's end return nothing and touch no memory.  28
+// ids a thread and round, us for 32 rows against 24 and 32, top_p alone: 4100 ids
+// 24.6 / 24.3 / 25.0, 26000 28.2 / 29.6 / 28.5, 50257 33.5 / 34.8 / 34.2, 131072
+// 70.5 / 70.8 / 69.2.
 __device__ __forceinline__ void gather_ranges(const float* src, int n, float a0, float a1, float b0,
                                               float b1, TopKShared& tk) {
-  constexpr int UN = AKH_GATHER_U;
+  constexpr int UN = 28;
   if (threadIdx.x == 0) tk.n_cand = 0;
   __syncthreads();
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>(src), (short)0, n * 4, 0x00020000);
   for (int c0 = 0; c0 < n; c0 += NT * UN) {
     const int i0 = c0 + (int)threadIdx.x;
     float v[UN];
 #pragma unroll
-    for (int u = 0; u < UN; ++u) v[u] = src[min(i0 + u * NT, n - 1)];
+    for (int u = 0; u < UN; ++u)
+      v[u] = __builtin_bit_cast(
+          float, __builtin_amdgcn_raw_buffer_load_b32(rs, (i0 + u * NT) * 4, 0, 0));
     uint32_t hits = 0;
 #pragma unroll
     for (int u = 0; u < UN; ++u)
@@ -532,7 +536,7 @@ __device__ __forceinline__ void gather_ranges(const float* src, int n, float a0,
     while (hits) {
       const int i = i0 + (__ffs((int)hits) - 1) * NT;
       hits &= hits - 1;
-      if (i >= n) break;
+      if (i >= n) break;  // zeros past the end
       const uint32_t slot = atomicAdd(&tk.n_cand, 1u);
       if (slot < (uint32_t)CCAP)
         tk.comp[slot] = ((unsigned long long)order_key(src[i]) << 32) | (0xFFFFFFFFu - (uint32_t)i);

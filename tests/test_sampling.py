@@ -160,16 +160,18 @@ def test_device_sampler_split_rows_edge_cases(backend, pkg, ora, rows, k):
 
 # Short rows, never binned; rows around the shortest that is (4100 ids: one part
 # that fills its workspace) and around the shortest that is binned for a
-# temperature alone (8200 ids, 7800 of more than 128 rows, 5500 of more than 256); over several parts
-# with a ragged last one (16 parts: 66001), and more rows than blocks of bins, with
-# one part and with two; in each: no top_k, top_k above and below what a bin
+# temperature alone (8200 ids, 7800 of more than 128 rows, 5500 of more than
+# 256); over several parts with a ragged last one (16 parts: 66001), and more rows
+# than blocks of bins, with one part and with two; rows of one gather round and
+# of one id more (28672).  In each: no top_k, top_k above and below what a bin
 # holds, a row of equal logits (every id in one bin: the radix path), one finite
 # logit, steps of ties, a far lower half, draws at both ends of [0, 1) and a grid
 # far finer and far coarser than the logits.
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows,n", [(7, 2049), (7, 2050), (7, 4101), (9, 20003), (300, 2500),
                                     (7, 4099), (7, 4100), (7, 8199), (7, 8200), (7, 66001),
-                                    (129, 7799), (129, 7800), (300, 5499), (300, 5500), (260, 33001), (800, 4100)])
+                                    (7, 28672), (7, 28673), (129, 7799), (129, 7800),
+                                    (300, 5499), (300, 5500), (260, 33001), (800, 4100)])
 @pytest.mark.parametrize("t,k,p", [(0.8, 0, 0.95), (1.0, 0, 1.0), (0.01, 0, 0.5), (50.0, 0, 0.3),
                                    (0.7, 1, 0.9), (1.2, 1000, 0.99), (0.9, 2000, 0.8)])
 def test_device_sampler_binned_rows(backend, pkg, ora, rows, n, t, k, p):
