@@ -1244,8 +1244,12 @@ akh_status ensure_prefill(akh_session* s, size_t rows) {
   HIP_TRY(hipMalloc(&s->pq, rows * d * 4));
   HIP_TRY(hipMalloc(&s->pattn, split_rows_f16_bytes(rows, (int)d)));
   HIP_TRY(hipMalloc(&s->pffn, split_rows_f16_bytes(rows, (int)F)));
-  HIP_TRY(hipMalloc(&s->pparts, kGemmPartsFloats * 4));
-  if (d > (size_t)kNormPartsMax) HIP_TRY(hipMalloc(&s->pwide, rows * d * 4));
+  if (split_capable(s->m->cfg)) {  // what only the split-fp16 kernels use
+    if (d <= (size_t)kNormPartsMax)
+      HIP_TRY(hipMalloc(&s->pparts, std::min(kGemmPartsFloats, kGemmPartsMax * rows * d) * 4));
+    else
+      HIP_TRY(hipMalloc(&s->pwide, rows * d * 4));
+  }
   HIP_TRY(hipMalloc(&s->ptok, rows * 4));
   HIP_TRY(hipMalloc(&s->p_at, (s->B + 1) * sizeof(int)));
   HIP_TRY(hipMalloc(&s->p_map, rows * sizeof(int2)));

@@ -11,8 +11,7 @@ the oracle (identical tokens, logits within 1e-3), also with the bfloat16 KV
 cache (within 2e-2) and through generate's sampler.
 """
 
-import dataclasses
-
+import ctypes
 import dataclasses
 
 import numpy as np
@@ -220,3 +219,30 @@ def test_few_sequences_long_ffn_matches_oracle(backend, pkg, ora, batch, dim, ff
         want = [r.decode_step(int(t)) for r, t in zip(refs, nxt)]
         logits, nxt = s.decode_step(None)
     s.close()
+
+
+def test_prefill_memory_is_what_its_rows_need(backend, pkg):
+    # 64 rows of dim 36 (no split kernels) and of dim 64 (eight K ranges of 64 x 64
+    # sums, 128 KB): a fixed 16 MB buffer of partial sums shows in either.
+    rt = ctypes.CDLL("libamdhip64.so")
+
+    def free():
+        backend.synchronize()
+        f, t = ctypes.c_size_t(), ctypes.c_size_t()
+        assert rt.hipMemGetInfo(ctypes.byref(f), ctypes.byref(t)) == 0
+        return f.value
+
+    for dim in (36, 64):
+        cfg = pkg.ModelConfig.new(97, dim, 1, 2, 64)
+        model = pkg.hip.Model(backend, cfg)
+        model.upload(pkg.synthetic_weights(cfg, seed=3))
+        sessions = [pkg.hip.Session(model, 64, 1) for _ in range(4)]
+        t = pkg.synthetic_tokens(64, 97, seed=4).reshape(1, -1)
+        sessions[0].prefill(t)
+        before = free()
+        for s in sessions[1:]:
+            s.prefill(t)
+        assert before - free() < 3 * (16 << 20), dim
+        for s in sessions:
+            s.close()
+        model.close()
