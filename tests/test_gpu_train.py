@@ -244,3 +244,32 @@ def test_forward_h3_grids_match_fp32_mfma(backend, pkg, batch, seq, dim, ffn):
     assert np.abs(hh - f.hidden()).max() < 2 * tol  # two layers
     assert np.abs(lh - lf).max() < 4 * tol  # the lm_head on rows scaled by the norm
     f.close()
+
+
+# Rows wider than 2048, where the norm that writes fp16 planes holds eight octets
+# a lane (with K ranges' partial sums to add, and without), and wider than
+# 4096, where fp32 rows are normed and converted.
+@pytest.mark.parametrize("batch,seq,dim,heads,ffn", [
+    (1, 40, 2056, 257, 520), (1, 300, 2304, 36, 1032), (2, 150, 4096, 64, 520),
+    (3, 700, 2304, 18, 264), (1, 70, 4104, 76, 520),
+])
+def test_forward_h3_wide_rows_match_fp32_mfma(backend, pkg, batch, seq, dim, heads, ffn):
+    M = pkg.hip.Model
+    cfg = dataclasses.replace(pkg.ModelConfig.new(97, dim, heads, 1, seq), ffn_hidden=ffn)
+    std = 0.02 * np.sqrt(64 / dim)
+    model = M(backend, cfg)
+    model.upload(pkg.synthetic_weights(cfg, seed=71, std=std))
+    assert model.prefill_split() == M.SPLIT_H3
+    toks = pkg.synthetic_tokens(batch * seq, 97, seed=72)
+    tgts = pkg.synthetic_tokens(batch * seq, 97, seed=73)
+    f = pkg.hip.Forward(model, batch, seq)
+    _, lh = f.loss(toks, tgts)
+    hh = f.hidden()
+    model.set_prefill_split(M.SPLIT_NONE)
+    _, lf = f.loss(toks, tgts)
+    # As above, with sum |a b| of a normed row (mean |a| 0.8) and a column N(0, std).
+    tol = 2 * (0.64 * dim * std) * (2.0 ** -22 + np.sqrt(dim) * 2.0 ** -24)
+    assert np.abs(hh - f.hidden()).max() < 2 * tol
+    assert np.abs(lh - lf).max() < 4 * tol
+    f.close()
+    model.close()

@@ -138,10 +138,9 @@ def test_device_sampler_matches_oracle(backend, pkg, ora, t, k, p, pen, ties):
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows,k", [(4, 40), (64, 40), (3, 200)])
 def test_device_sampler_split_rows_edge_cases(backend, pkg, ora, rows, k):
-    # run_chat's parameters with rows split over parts of the vocabulary (16
-    # parts at 4 rows, 4 at 64; top_k 200 at 3 rows: 10 parts, so that all
-    # parts' top_k fit the merge): a quarter of the vocabulary at -inf (parts
-    # with no finite element), only 10 finite logits (fewer than top_k: the
+    # run_chat's parameters with rows binned by several blocks (12 parts of the
+    # vocabulary at 3 and 4 rows, 4 at 64): a quarter of the vocabulary at -inf
+    # (parts with no finite element), only 10 finite logits (fewer than top_k: the
     # radix path), integer logits (ties across parts, lower index first),
     # and plain rows; every row against the oracle.
     rng = np.random.default_rng(77 + rows)
