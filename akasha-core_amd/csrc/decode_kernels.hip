@@ -1475,7 +1475,7 @@ __global__ __launch_bounds__(256) void k_dec_few(DecFewParams p) {
           v.z += f * o[sp].z;
           v.w += f * o[sp].w;
         }
-        const float inv = 1.0f / L;
+        const float inv = L > 0.f ? 1.0f / L : 0.f;  // 0: every score at -inf
         v = make_float4(v.x * inv, v.y * inv, v.z * inv, v.w * inv);
       } else {
 #pragma unroll

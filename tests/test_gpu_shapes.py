@@ -246,3 +246,24 @@ def test_prefill_memory_is_what_its_rows_need(backend, pkg):
         for s in sessions:
             s.close()
         model.close()
+
+
+def test_few_sequences_scores_at_minus_infinity(backend, pkg):
+    # A first token whose one score overflows to -inf (q columns 1e20, k columns
+    # -1e20 times the same sum): no weight remains and the attention adds nothing,
+    # on the few-sequence and on the batched kernels alike.
+    cfg = pkg.ModelConfig.new(97, 64, 2, 1, 16)
+    w = pkg.synthetic_weights(cfg, seed=31)
+    w[2][:, :64] = 1e20
+    w[2][:, 64:128] = -1e20
+    model = pkg.hip.Model(backend, cfg)
+    model.upload(w)
+    out = []
+    for batch in (1, 5):
+        s = pkg.hip.Session(model, 16, batch)
+        logits, _ = s.decode_step(np.full(batch, 11, np.uint32))
+        out.append(logits[0].copy())
+        s.close()
+    assert np.isfinite(out[1]).all()
+    np.testing.assert_allclose(out[0], out[1], atol=1e-5)
+    model.close()
