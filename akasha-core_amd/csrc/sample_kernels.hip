@@ -491,7 +491,8 @@ __device__ void reduce_counts(const uint32_t (&c)[NTH], uint32_t base, TopKShare
 }
 
 // The smallest float whose grid cell is at least `cell` (floor(l * scale),
-// which grows with l).
+// which grows with l; |cell| <= 2^30 and 2 <= scale <= 2^60, so the quotient is
+// at most a few floats away and -2^-149 already lies in cell -1).
 __device__ __forceinline__ float cell_low(float cell, float scale) {
   auto at_least = [&](float l) { return floorf(__fmul_rn(l, scale)) >= cell; };
   auto step = [](float l, int by) {  // the by-th float above or below l
@@ -738,25 +739,34 @@ __host__ __device__ constexpr long hist_doubles(int parts) { return (long)parts 
 // an id, of the workspace's 8).
 constexpr int kHistMin = 2 * (kBins + 2);
 
-// Cells per logit: 64, or 48 per unit of l / T where that is finer (cells of
-// ~150 ids at the densest of 50257 logits N(0, 2^2); 2047 cells reach 42 T below
-// the maximum, e^-42 of its weight, or 32), or finer still on a flat row,
-// whose logits would share a few cells: 800 to the range lo .. hi of 1024 of the
-// row's logits, which is about 6.5 standard deviations (32 rows x 50257 N(0,
+// Cells per logit.  For weights 64, or 48 per unit of l / T where that is finer
+// (cells of ~150 ids at the densest of 50257 logits N(0, 2^2); 2047 cells reach 42
+// T below the maximum, e^-42 of its weight, or 32), or finer still on a flat
+// row, whose logits would share a few cells: 800 to the range lo .. hi of 1024 of
+// the row's logits, which is about 6.5 standard deviations (32 rows x 50257 N(0,
 // 0.01^2) on MI355X, us without / with: top_k 40 108 / 23, top_p alone 173 / 36).
+// For counts, which no temperature enters, 800 to that range or 4 (with a mask's
+// value in it, 2047 cells still reach 512): 32 rows of N(0, 20^2) with top_k 40
+// 31 us, 66 on the weights' grid, whose end lies above the 40th.
 // No finer than keeps hi's cell at 2^23, so that a large maximum's cells are
-// exact (far below zero hi is a mask's value and says nothing of the maximum).
-__device__ __forceinline__ float grid_scale(float temperature, float hi, float lo) {
-  float s = fmaxf(64.0f, 48.0f / temperature);
-  if (hi > lo) s = fmaxf(s, 800.0f / (hi - lo));
-  if (hi > -1e4f && hi < INFINITY) s = fminf(s, 0x1p23f / fabsf(hi));
+// exact (far below zero hi is a mask's value and says nothing of the maximum,
+// beyond 2^22 a cell would be wider than a logit).  From 2 to 2^60: every float
+// but 0 has a cell other than 0's, which cell_low's steps rely on.
+inline float grid_base(float temperature, bool count) {
+  return count ? 4.0f : fmaxf(64.0f, 48.0f / temperature);
+}
+__device__ __forceinline__ float grid_scale(float base, float hi, float lo) {
+  float s = hi > lo ? fmaxf(base, 800.0f / (hi - lo)) : fmaxf(base, 64.0f);
+  if (hi > -1e4f && hi <= 0x1p22f) s = fminf(s, 0x1p23f / fabsf(hi));
   return fminf(s, 0x1p60f);
 }
 __device__ __forceinline__ float grid_cell(float l, float scale) {
   return floorf(__fmul_rn(l, scale));
 }
 
-__global__ __launch_bounds__(NT) void k_sample_hist(SampleArgs a) {
+// `base_scale`: grid_base.  58 registers, so two blocks share a CU (with 86, 512 x 131072
+// took 444 us with run_chat's parameters instead of 315).
+__global__ __launch_bounds__(NT) void k_sample_hist(SampleArgs a, float base_scale) {
   extern __shared__ uint32_t bitmap[];
   __shared__ SampleShared sh;
   const int m = blockIdx.x, part = blockIdx.y, parts = gridDim.y;
@@ -824,7 +834,7 @@ __global__ __launch_bounds__(NT) void k_sample_hist(SampleArgs a) {
     nlo = fmaxf(nlo, r.y);
     nans |= sh.wave_u[k];
   }
-  const float scale = grid_scale(a.temperature, hi, -nlo);
+  const float scale = grid_scale(base_scale, hi, -nlo);
   const bool empty = mx == -INFINITY, bad = nans || mx == INFINITY;
   double own = 0.0;
   if (!bad && !empty) {
@@ -1233,7 +1243,8 @@ hipError_t launch_sample_rows(const SampleArgs& a, int rows, hipStream_t s) {
     parts = std::max(AKH_SAMPLE_BLOCKS / rows, std::min((a.n + 32767) / 32768, 1024 / rows));
     parts = std::min(kPartsMax, std::max(1, parts));
     while (parts > 1 && (2 * hist_doubles(parts) > a.n || a.n / parts < NT)) --parts;
-    hipLaunchKernelGGL(k_sample_hist, dim3(rows, parts), dim3(NT), lds, s, a);
+    hipLaunchKernelGGL(k_sample_hist, dim3(rows, parts), dim3(NT), lds, s, a,
+                       grid_base(a.temperature, a.top_k > 0 && a.top_k < a.n));
   }
   hipLaunchKernelGGL(k_sample_rows, dim3(rows), dim3(NT), lds, s, a, parts);
   return hipGetLastError();

@@ -231,10 +231,11 @@ def test_device_sampler_largest_vocabulary_with_penalty(backend, pkg, ora, t, k,
 
 # Binned rows whose grid follows their logits: flat ones (down to a range of a
 # few floats, and all equal), half of the ids or all but eight at a mask's value,
-# a grid capped by large logits, and the same 1024 ids being all masked.
+# a grid capped by large logits, the same 1024 ids being all masked, and logits
+# that spread beyond the bins.
 @pytest.mark.gpu
 @pytest.mark.parametrize("t,k,p", [(0.8, 40, 0.95), (0.8, 0, 0.95), (1.0, 0, 1.0), (1e-4, 40, 0.9),
-                                   (1e-4, 0, 0.9), (0.7, 1000, 0.99)])
+                                   (1e-4, 0, 0.9), (0.7, 1000, 0.99), (0.05, 64, 1.0)])
 def test_device_sampler_binned_rows_flat_and_masked(backend, pkg, ora, t, k, p):
     rows, n = 12, 20003
     rng = np.random.default_rng(11)
@@ -251,6 +252,7 @@ def test_device_sampler_binned_rows_flat_and_masked(backend, pkg, ora, t, k, p):
     l[8] = g[8] * 1e5
     l[9] = 1e8 + g[9] * 100
     l[10] = np.float32(1e-42) * np.round(g[10])
+    l[11] = g[11] * 200
     u = rng.random(rows)
     seen_rows = [rng.integers(0, n, 40).astype(np.uint32) for _ in range(rows)]
     for pen in (1.0, 1.15):
