@@ -21,7 +21,7 @@
 // of the seen ids in LDS.
 //
 // Rows of at least kHistMin ids skip that: a first kernel spreads each row
-// over several blocks, which bin their part's logits on a fixed grid (2047
+// over several blocks, which bin their part's logits on the row's grid (2047
 // bins below the part's maximum) and sum each bin's f64 weights, or count its
 // elements where 0 < top_k <= 1024.  The row's block adds the parts' bins,
 // finds the bins in which the cuts fall, gathers their members (a few hundred
@@ -29,10 +29,11 @@
 // exactly there.  With top_k that list is the top_k, which then goes through
 // the reference's own sequence: f64 probabilities summed in order, the top_p
 // prefix, the walk r -= p.  NaN, an infinite maximum, cuts below the bins and
-// bins of too many ids (ties) take the radix path.
-// Shorter rows with 0 < top_k <= 1024: a cut on d = max - l admitting between
-// top_k and 2048 elements is found by counting against 16 thresholds per pass
-// (powers of four, then 16-way refinements) instead of the bins.
+// bins of too many ids (ties) are left to the other paths.
+// Shorter rows, and those the bins leave, with 0 < top_k <= 1024: a cut on d = max
+// - l admitting between top_k and 2048 elements is found by counting against 16
+// thresholds per pass (powers of four, then 16-way refinements); where that
+// fails too, the radix path.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -1066,8 +1067,8 @@ __global__ __launch_bounds__(NT) void k_sample_rows(SampleArgs a, int parts) {
   const uint32_t* bm = pick < (uint32_t)n ? nullptr : seen_bitmap(a, seen, bitmap);
   auto key_of = [&](int i) { return order_key(pen_logit(row, i, bm, a.penalty)); };
   auto l_at = [&](int i) { return pen_logit(row, i, bm, a.penalty); };
-  if (parts <= 0 && a.temperature > 0.0f && a.top_k > 0 && a.top_k < n && a.top_k <= KCAP &&
-      topk_candidates(n, l_at, (uint32_t)a.top_k, sh, tk) >= 0)
+  if (pick >= (uint32_t)n && a.temperature > 0.0f && a.top_k > 0 && a.top_k < n &&
+      a.top_k <= KCAP && topk_candidates(n, l_at, (uint32_t)a.top_k, sh, tk) >= 0)
     pick = tail_topk((uint32_t)a.top_k, a.temperature, a.top_p, r, tk);
   const bool picked = pick < (uint32_t)n;
   if (picked) {
@@ -1234,7 +1235,7 @@ hipError_t launch_sample_rows(const SampleArgs& a, int rows, hipStream_t s) {
                    : rows > 128      ? 7800
                                      : 2 * kHistMin;
   int parts = 0;
-  if (a.temperature > 0.0f && a.n >= from && (a.top_k <= KCAP || a.top_k >= a.n)) {
+  if (a.temperature > 0.0f && a.temperature < INFINITY && a.n >= from && (a.top_k <= KCAP || a.top_k >= a.n)) {
     // Parts for about 256 blocks of bins in all, at most 16 a row, and no part
     // above 32768 ids while there are at most 1024 blocks (top_k 40 with top_p and
     // a penalty, us at 1, 2, 4 and 8 parts: 256 x 131072 236, 169, 157, 144; 256 x

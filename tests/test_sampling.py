@@ -259,3 +259,18 @@ def test_device_sampler_binned_rows_flat_and_masked(backend, pkg, ora, t, k, p):
         got = _device_sample(pkg, backend, l, t, k, p, pen, seen_rows, u)
         want = [ora.sample_token(l[i], t, k, p, seen_rows[i], pen, u[i]) for i in range(rows)]
         assert list(got) == want, pen
+
+
+# Weights of NaN: at an infinite temperature an id at -inf has one, and the
+# last id of the order is what is left, as in the reference.
+@pytest.mark.gpu
+@pytest.mark.parametrize("k,p", [(0, 0.95), (0, 1.0), (40, 0.9), (3000, 0.9)])
+def test_device_sampler_infinite_temperature(backend, pkg, ora, k, p):
+    rng = np.random.default_rng(3)
+    l = (rng.standard_normal((4, 9001)) * 2.5).astype(np.float32)
+    l[0, ::2] = -np.inf
+    l[1, 7:] = -np.inf
+    l[2, :4096] = -np.inf
+    u = rng.random(4)
+    got = _device_sample(pkg, backend, l, np.inf, k, p, 1.0, [[]] * 4, u)
+    assert list(got) == [ora.sample_token(l[i], np.inf, k, p, [], 1.0, u[i]) for i in range(4)]
