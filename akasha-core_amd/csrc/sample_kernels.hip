@@ -1120,7 +1120,9 @@ __global__ __launch_bounds__(NT) void k_sample_rows(SampleArgs a, int parts) {
     uint32_t last = kth < (uint32_t)n ? kth : (uint32_t)n;  // last kept element, n = unknown
     if (a.top_p < 1.0f) {
       // No crossing keeps every element (and still renormalises).
-      const uint32_t cut = select_desc(n, key_of, w, (double)a.top_p * sum, true, sh);
+      // A target of zero or less is met by the first element, not by an empty bin.
+      const double want = (double)a.top_p * sum;
+      const uint32_t cut = select_desc(n, key_of, w, want <= 0.0 ? 0x1p-1074 : want, true, sh);
       const uint32_t ckey = cut < (uint32_t)n ? key_of((int)cut) : 0u;
       double kept = 0.0;
       for (int i = threadIdx.x; i < n; i += NT) {

@@ -274,3 +274,21 @@ def test_device_sampler_infinite_temperature(backend, pkg, ora, k, p):
     u = rng.random(4)
     got = _device_sample(pkg, backend, l, np.inf, k, p, 1.0, [[]] * 4, u)
     assert list(got) == [ora.sample_token(l[i], np.inf, k, p, [], 1.0, u[i]) for i in range(4)]
+
+
+# A top_p of zero or less keeps the first id, on every path: a short row, a binned
+# one, and the radix path behind the bins (equal logits, top_k above 1024).
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [500, 5000])
+@pytest.mark.parametrize("k", [0, 40, 2000])
+@pytest.mark.parametrize("p", [0.0, -1.0])
+def test_device_sampler_top_p_zero_is_greedy(backend, pkg, ora, n, k, p):
+    rng = np.random.default_rng(n + k)
+    l = (rng.standard_normal((4, n)) * 2.5).astype(np.float32)
+    l[0] = 0.5
+    l[1] *= 1e4
+    l[2] = np.round(l[2])
+    u = rng.random(4)
+    got = _device_sample(pkg, backend, l, 0.8, k, p, 1.0, [[]] * 4, u)
+    assert list(got) == [ora.sample_token(l[i], 0.8, k, p, [], 1.0, u[i]) for i in range(4)]
+    assert list(got) == list(np.argmax(l, axis=1))
