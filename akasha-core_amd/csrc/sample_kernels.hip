@@ -748,7 +748,7 @@ constexpr int kHistMin = 2 * (kBins + 2);
 // 0.01^2) on MI355X, us without / with: top_k 40 108 / 23, top_p alone 173 / 36).
 // For counts, which no temperature enters, 800 to that range or 4 (with a mask's
 // value in it, 2047 cells still reach 512): 32 rows of N(0, 20^2) with top_k 40
-// 31 us, 66 on the weights' grid, whose end lies above the 40th.
+// 21 us, 66 on the weights' grid, whose end lies above the 40th.
 // No finer than keeps hi's cell at 2^23, so that a large maximum's cells are
 // exact (far below zero hi is a mask's value and says nothing of the maximum,
 // beyond 2^22 a cell would be wider than a logit).  From 2 to 2^60: every float
@@ -1187,8 +1187,8 @@ size_t sample_scratch_bytes(int rows, int n) { return (size_t)rows * n * sizeof(
 // weights, kNoAllocSampleElems doubles = 16 MiB).  Every GPU the library
 // runs on holds its own copy until the process ends.  In host code the
 // array's name is not a device address: kernels get the address from
-// sample_noalloc_scratch().  k_sample_rows writes every weight it reads
-// within the same launch, so the array needs no clearing between calls.
+// sample_noalloc_scratch().  A call's kernels write every bin, header and
+// weight they read, so the array needs no clearing between calls.
 namespace {
 __device__ __align__(256) double scratch[kNoAllocSampleElems];
 std::mutex g_scratch_mu;

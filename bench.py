@@ -550,7 +550,8 @@ def sampler_measurement(hip, be, reps=20):
     seen_len = be.tensor(np.full(rows, H, np.uint32))
     uni = be.tensor(rng.random(rows))
     out = be.zeros(rows, np.uint32)
-    res = {"workload": f"{rows} rows x {n} logits, {H} seen ids per row, one launch per call"}
+    res = {"workload": f"{rows} rows x {n} logits, {H} seen ids per row, "
+                       "two launches per call (greedy: one)"}
     for name, kw in (("run_chat", dict(temperature=0.8, top_k=40, top_p=0.95, repetition_penalty=1.15)),
                      ("top_k_40", dict(temperature=0.8, top_k=40)),
                      ("top_p_0.95", dict(temperature=0.8, top_p=0.95)),
